@@ -421,6 +421,21 @@ int logo_add_rmsnorm(const void* r, const void* x, const void* w, void* s_out, v
 int logo_silu_mul(const void* gu, int64_t ld, void* y, int64_t rows, int cols, int dtype, void* stream);
 
 /*
+ * A linear layer of a decode step, y = x W^T for m <= 16 rows x [m, k] (row
+ * stride ldx, a multiple of 8) and W [n, k] (k a multiple of 32; x, w and
+ * norm_w 16-byte aligned), with its neighbours in the decoder fused in:
+ *   norm_w != NULL (k <= 2048): x is RMS-normalised first (as logo_rmsnorm);
+ *   resid != NULL [m, n]: y = resid + x W^T, the product rounded to bf16 first;
+ *   glu != 0: W is [2 n, k], gate rows then up rows, and y [m, n] is
+ *     silu(x Wg^T) * x Wu^T with logo_silu_mul's rounding.
+ * Sums are fp32 in a fixed order.  Replaces, at decode, the projections of
+ * logo/layers/logo.py:112-130 and logo/modules/mlp.py:24-27 with the norms
+ * and residual adds of logo/modeling_logo.py:58-66.
+ */
+int logo_dec_linear(const void* x, int64_t ldx, const void* w, const void* norm_w, float eps, const void* resid,
+                    void* y, int m, int n, int k, int glu, int dtype, void* stream);
+
+/*
  * RMSNorm of rows [rows, cols] bf16 with weight [cols]: y = w * bf16(x *
  * rsqrt(mean(x^2) + eps)), mean in fp32 (logo/modules/layernorm.py:17-22; the
  * decoder's input / post-attention / final norms, logo/modeling_logo.py:58-59,

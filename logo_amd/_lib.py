@@ -57,6 +57,7 @@ SIGNATURES = {
     "logo_rope": ([_P, _P, _I, _P, _P, _I, _P, _P, _I, _P, _P, _I, _P, _P, _I64, _I, _I, _I, _P], _I),
     "logo_rmsnorm": ([_P, _P, _P, _I64, _I, _F, _I, _P], _I),
     "logo_add_rmsnorm": ([_P, _P, _P, _P, _P, _I64, _I, _F, _I, _P], _I),
+    "logo_dec_linear": ([_P, _I64, _P, _P, _F, _P, _P, _I, _I, _I, _I, _I, _P], _I),
     "logo_silu_mul": ([_P, _I64, _P, _I64, _I, _I, _P], _I),
     "logo_head_proj": ([_P, _P, _P, _I, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _P], _I),
     "logo_decode_qkv": ([_P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _I, _I, _I, _I, _I, _I64,

@@ -281,6 +281,10 @@ constexpr int kBufRsrcWord3 = 0x00020000;  // raw, untyped 32-bit buffer (gfx9 f
 __device__ __forceinline__ void buf_load_lds16(__amdgpu_buffer_rsrc_t r, bf16* lds, uint32_t voff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
 }
+// The same as a streaming (non-temporal) load, for data read once.
+__device__ __forceinline__ void buf_load_lds16_nt(__amdgpu_buffer_rsrc_t r, bf16* lds, uint32_t voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 2);
+}
 
 template <int D, int NW = 4>
 struct TileBufDma {

@@ -29,7 +29,7 @@ import torch.nn.functional as F
 
 from .ops.decode import LogoKVCache, decode_attn, decode_attn_fused, decode_qkv
 from .ops.epilogue import logo_epilogue
-from .ops.glue import attn_inputs, head_linear, head_proj, rms_norm, rope, rope_apply_
+from .ops.glue import attn_inputs, dec_linear, dec_linear_ok, head_linear, head_proj, rms_norm, rope, rope_apply_
 from .ops.sq_attn import dense_causal_attn, sq_full_attn, swa_attn
 
 __all__ = ["LoGoConfig", "LoGoAttention", "Attention", "RMSNorm", "rope_cos_sin", "apply_rope", "position_ids_for"]
@@ -101,6 +101,28 @@ def _fused_ok(*tensors) -> bool:
     if any(t.requires_grad for t in tensors) and torch.is_grad_enabled():
         return False
     return all(t.is_cuda and t.dtype == torch.bfloat16 for t in tensors)
+
+
+def _unhooked(*modules) -> bool:
+    """Whether calling the modules' own arithmetic directly is what calling
+    them would do: no forward hook of theirs or of every module is skipped."""
+    return not torch.nn.modules.module._has_any_global_hook() and not any(
+        m._forward_hooks or m._forward_pre_hooks for m in modules)
+
+
+def _dec_weight_ok(rows: int, w) -> bool:
+    """Whether ``dec_linear`` serves ``rows`` input rows of a bias-free linear
+    layer with weight ``w`` (inference, outside autocast)."""
+    return (dec_linear_ok(rows, w) and _fused_ok(w) and not torch.is_autocast_enabled("cuda"))
+
+
+def linear_rows(lin: nn.Linear, x):
+    """``lin(x)``, on ``dec_linear`` for the few rows of a decode step."""
+    w = lin.weight
+    if type(lin) is nn.Linear and lin.bias is None and x.numel() <= 16 * x.shape[-1] and _fused_ok(x, w) \
+            and x.shape[-1] == w.shape[1] and _dec_weight_ok(x.numel() // x.shape[-1], w) and _unhooked(lin):
+        return dec_linear(x, w)
+    return lin(x)
 
 
 def position_ids_for(B: int, T: int, device, cu_seqlens=None, cache: Optional[LogoKVCache] = None):
@@ -362,12 +384,18 @@ class LoGoAttention(nn.Module):
         """Decode step with the stacked q / k / v / gate GEMM and one launch for
         the global projections, RoPE and cache appends (same arithmetic as the
         step-by-step path: the same roundings, in the same order)."""
-        B = hidden_states.shape[0]
+        w = self._decode_weight()
+        qkv = dec_linear(hidden_states, w) if _dec_weight_ok(hidden_states.shape[0], w) else F.linear(hidden_states, w)
+        return self._decode_rows(qkv, cache, position_embeddings, position_ids)
+
+    def _decode_rows(self, qkv, cache: LogoKVCache, position_embeddings, position_ids):
+        """A decode step from its stacked projection rows ``[B, 1, q | k | v |
+        gate]`` to the input ``[B, 1, H D]`` of o_proj and the gate."""
+        B = qkv.shape[0]
         H, HK, D = self.num_heads, self.num_key_value_heads, self.head_dim
-        qkv = F.linear(hidden_states, self._decode_weight()).view(B, -1)
+        qkv = qkv.view(B, -1)
         n_qkv = (H + 2 * HK) * D
-        cos, sin = _cos_sin(self, B, 1, hidden_states.device, qkv.dtype, position_ids, None, cache,
-                            position_embeddings)
+        cos, sin = _cos_sin(self, B, 1, qkv.device, qkv.dtype, position_ids, None, cache, position_embeddings)
         q, gq, gate = decode_qkv(qkv, self.q_global_proj, self.k_global_proj, self.v_global_proj, cos, sin, cache,
                                  self.layer_idx, H, HK, gate_col=n_qkv)
         gate = gate.view(B, 1, 1)
@@ -402,7 +430,7 @@ class LoGoAttention(nn.Module):
                     self.gate_avg.add_(gate.sum().float())
                     self.global_token_count.add_((gate >= self.gate_thres).sum().float())
                     self.total_token_count.add_(gate.numel())
-            return self.o_proj(out), None, past_key_value
+            return linear_rows(self.o_proj, out), None, past_key_value
         cs = lambda dtype: _cos_sin(self, B, T, hidden_states.device, dtype, position_ids,  # noqa: E731
                                     cu_seqlens, past_key_value, position_embeddings)
         cos = sin = None

@@ -21,10 +21,10 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .layers import (Attention, LoGoAttention, LoGoConfig, RMSNorm, _fused_ok, padding_mask, position_ids_for,
-                     rope_cos_sin)
+from .layers import (Attention, LoGoAttention, LoGoConfig, RMSNorm, _dec_weight_ok, _fused_ok, _unhooked, linear_rows,
+                     padding_mask, position_ids_for, rope_cos_sin)
 from .ops.decode import LogoKVCache
-from .ops.glue import add_rms_norm, silu_mul
+from .ops.glue import add_rms_norm, dec_linear, silu_mul
 
 __all__ = ["LoGoMLP", "LoGoDecoderLayer", "LoGoModel", "LoGoForCausalLM"]
 
@@ -71,6 +71,32 @@ class LoGoDecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
+    def _decode_ok(self, h, cache) -> bool:
+        """Whether a decode step of this layer runs as ``_decode_step``: plain
+        modules without hooks, few rows, bf16 inference."""
+        a, m = self.self_attn, self.mlp
+        norms = (self.input_layernorm, self.post_attention_layernorm)
+        if type(self) is not LoGoDecoderLayer or type(a) is not LoGoAttention or type(m) is not LoGoMLP \
+                or a.training or any(type(n) is not RMSNorm for n in norms):
+            return False
+        lins = (a.q_proj, a.k_proj, a.v_proj, a.gate_proj, a.o_proj, m.gate_proj, m.up_proj, m.down_proj)
+        if any(type(x) is not nn.Linear or x.bias is not None for x in lins) or m.up_proj.weight.shape[0] % 8:
+            return False
+        return (_unhooked(self, a, m, *norms, *lins) and a._fused_decode_ok(h, cache)
+                and _fused_ok(*(n.weight for n in norms), *(x.weight for x in lins))
+                and all(_dec_weight_ok(h.shape[0], x.weight) for x in (a.q_proj, a.o_proj, m.up_proj, m.down_proj)))
+
+    def _decode_step(self, h, cache: LogoKVCache, position_embeddings, position_ids):
+        """One decode step of ``h [B, 1, C]``: the same arithmetic as ``forward``,
+        each projection one launch with the norm, residual add or SwiGLU
+        beside it."""
+        a, n1, n2 = self.self_attn, self.input_layernorm, self.post_attention_layernorm
+        qkv = dec_linear(h, a._decode_weight(), norm_w=n1.weight, eps=n1.variance_epsilon)
+        out, _ = a._decode_rows(qkv, cache, position_embeddings, position_ids)
+        h = dec_linear(out, a.o_proj.weight, resid=h)
+        act = dec_linear(h, self.mlp._gate_up_weight(), norm_w=n2.weight, eps=n2.variance_epsilon, glu=True)
+        return dec_linear(act, self.mlp.down_proj.weight, resid=h)
+
     def forward(self, hidden_states, attention_mask=None, position_ids=None, cu_seqlens=None,
                 past_key_value: Optional[LogoKVCache] = None, position_embeddings=None):
         residual = hidden_states
@@ -112,6 +138,11 @@ class LoGoModel(nn.Module):
                                                                              past_key_value)
         # rotary cos / sin once for all layers (logo/modeling_logo.py:233-234)
         pe = rope_cos_sin(pos.expand(B, T), self.config.head_dim, self.config.rope_theta, h.dtype)
+        if T == 1 and past_key_value is not None and cu_seqlens is None and _fused_ok(h) and all(
+                layer._decode_ok(h, past_key_value) for layer in self.layers):
+            for layer in self.layers:
+                h = layer._decode_step(h, past_key_value, pe, position_ids)
+            return self.norm(h)
         if _fused_ok(h) and h.shape[-1] <= 4096:
             # inference: each residual add fused with the norm that follows it
             # (post-attention norm, the next layer's input norm, the final norm)
@@ -179,7 +210,7 @@ class LoGoForCausalLM(nn.Module):
                        past_key_value=past_key_value)
         if last_only:
             h = h[:, -1]
-        return self.lm_head(h)
+        return linear_rows(self.lm_head, h)
 
     @torch.no_grad()
     def prefill(self, input_ids, cache: LogoKVCache, attention_mask=None):

@@ -1,0 +1,79 @@
+"""The decode step's linear layers (``dec_linear``) against float64 products.
+
+Sizes at the edges of the kernel: one k step and uneven k ranges of its waves,
+one and several batches of steps, output columns that end inside a tile, one
+to sixteen rows, a strided input.  Every output is a few bf16 roundings away
+from the float64 result: of the product, of the normalised input (each input
+off by 2^-8 at most, in independent directions) and of the last operation.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _norm(x, w, eps):
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps) * w
+
+
+@pytest.mark.parametrize("m", [1, 5, 16])
+@pytest.mark.parametrize("n,k", [(8, 32), (40, 288), (24, 1024), (6152, 1056), (16, 2048), (48, 2080), (32, 5632),
+                                 (200, 4128)])
+@pytest.mark.parametrize("mode", ["plain", "norm", "resid", "glu", "norm_glu"])
+def test_dec_linear(gpu, m, n, k, mode):
+    from logo_amd.ops.glue import dec_linear
+
+    g = torch.Generator().manual_seed(m * n + k)
+    glu = mode.endswith("glu")
+    x = torch.randn(m, k + 8, generator=g).bfloat16().to(gpu)[:, :k]  # rows apart by more than k
+    w = (torch.randn(2 * n if glu else n, k, generator=g) / k ** 0.5).bfloat16().to(gpu)
+    nw = (1 + 0.1 * torch.randn(k, generator=g)).bfloat16().to(gpu) if mode.startswith("norm") else None
+    if nw is not None and k > 4096:
+        pytest.skip("the norm launch takes at most 4096 columns")
+    res = torch.randn(m, n, generator=g).bfloat16().to(gpu) if mode == "resid" else None
+    got = dec_linear(x, w, norm_w=nw, eps=1e-5, resid=res, glu=glu).double()
+    xd = x.double() if nw is None else _norm(x.double(), nw.double(), 1e-5)
+    y = xd @ w.double().T
+    # rounding of one product: its own, and that of its normalised inputs
+    u = 2.0 ** -8
+    tol = u * y.abs() + 1e-5
+    if nw is not None:
+        tol = tol + 6 * 2 * u * (xd.pow(2) @ w.double().T.pow(2)).sqrt()
+    if glu:
+        ya, yb = y.split(n, dim=1)
+        ta, tb = tol.split(n, dim=1)
+        s = torch.nn.functional.silu(ya)
+        ref = s * yb
+        # |silu'| <= 1.1
+        tol = (1.1 * ta + u * s.abs()) * (yb.abs() + tb) + (s.abs() + 1.1 * ta) * tb + u * ref.abs() + 1e-5
+    else:
+        ref = y if res is None else y + res.double()
+        tol = tol + u * ref.abs()
+    assert got.shape == ref.shape
+    assert bool(((got - ref).abs() <= tol).all()), f"max excess {float(((got - ref).abs() - tol).max()):.3e}"
+
+
+def test_hooks_and_other_modules_keep_their_calls(gpu):
+    """A decode step calls a module that carries a forward hook (or is no plain
+    linear layer) as before, with the same logits within bf16 rounding."""
+    from logo_amd.layers import LoGoConfig
+    from logo_amd.model import LoGoForCausalLM
+
+    cfg = LoGoConfig(vocab_size=256, hidden_size=256, intermediate_size=512, num_hidden_layers=2,
+                     num_attention_heads=4, gate_thres_init=-1.0)
+    model = LoGoForCausalLM(cfg)
+    model.init_weights(torch.Generator().manual_seed(0))
+    model = model.to(device=gpu, dtype=torch.bfloat16).eval()
+    ids = torch.randint(0, 256, (3, 40), generator=torch.Generator().manual_seed(1)).to(gpu)
+    tok = ids[:, 0].clone()
+    logits, calls = [], []
+    for hooked in (False, True):
+        cache = model.new_cache(3, 60, device=gpu)
+        model.prefill(ids, cache)
+        if hooked:
+            for mod in (model.model.layers[0].mlp, model.model.layers[1].self_attn.o_proj, model.lm_head):
+                mod.register_forward_hook(lambda *a: calls.append(1))
+        logits.append(model.decode_step(tok, cache).double())
+    assert len(calls) == 3
+    assert float((logits[0] - logits[1]).norm() / logits[1].norm()) <= 2e-2
