@@ -171,6 +171,13 @@ size_t logo_sq_workspace_bytes(int64_t n_tokens, int nseq, int hq, int d);
 size_t logo_sq_workspace_counter_bytes(void);
 
 /*
+ * The same for head dim 256 in bf16 / fp16 without a window (whose kernels
+ * logo_sq_workspace_bytes does not count): with a workspace of this size, its
+ * counters zero, the forward and dq of that head dim split too.
+ */
+size_t logo_sq_wide_workspace_bytes(int hq);
+
+/*
  * 1 when calls with head dim d and element type dtype run on the generic
  * attention kernels (d = 256, or LOGO_DTYPE_F32), 0 for the tuned ones (no
  * counterpart in the reference, whose Triton kernels take every size).  The

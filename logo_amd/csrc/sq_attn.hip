@@ -206,6 +206,8 @@ extern "C" size_t logo_sq_workspace_bytes(int64_t n_tokens, int nseq, int hq, in
   return part == 0 ? 0 : split_cnt_bytes() + part;
 }
 
+extern "C" size_t logo_sq_wide_workspace_bytes(int hq) { return hq < 1 ? 0 : wide_workspace_bytes(hq); }
+
 extern "C" size_t logo_sq_workspace_counter_bytes(void) { return split_cnt_bytes(); }
 
 extern "C" int logo_sq_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -224,6 +226,7 @@ extern "C" int logo_sq_fwd(const void* q, const void* k, const void* v, void* o,
   a.ws_bytes = workspace ? workspace_bytes : 0;
   const bool sparse = q_idx != nullptr;
   const bool win = window >= 0;
+  if (wide_applies(a, d, dtype)) return wide_launch(a, as_stream(stream), kWideFwd, sparse, dtype == LOGO_DTYPE_F16);
   if (gen_applies(d, dtype)) return gen_launch_fwd(a, as_stream(stream), d, dtype, sparse);
   return sq_launch_fwd(a, as_stream(stream), d, sparse, win, dtype == LOGO_DTYPE_F16);
 }
@@ -268,16 +271,18 @@ static int bwd_entry(LOGO_BWD_PARAMS, int phase) {
   const bool win = window >= 0;
   const bool half = dtype == LOGO_DTYPE_F16;
   hipStream_t st = as_stream(stream);
-  if (generic) {  // the generic kernels read q and dO in place (no compacted copies)
+  if (generic) {  // these kernels read q and dO in place (no compacted copies)
+    const bool wide = wide_applies(a, d, dtype);
     if (phase < 0 || phase == 0) {
-      rc = gen_launch_delta(a, st, d, dtype, sparse);
+      rc = wide ? wide_launch(a, st, kWideDelta, sparse, half) : gen_launch_delta(a, st, d, dtype, sparse);
       if (rc != LOGO_OK) return rc;
     }
     if (phase < 0 || phase == 1 || phase == 3) {
-      rc = gen_launch_dq(a, st, d, dtype, sparse);
+      rc = wide ? wide_launch(a, st, kWideDq, sparse, half) : gen_launch_dq(a, st, d, dtype, sparse);
       if (rc != LOGO_OK) return rc;
     }
-    if (phase < 0 || phase == 2 || phase == 3) rc = gen_launch_dkv(a, st, d, dtype, sparse);
+    if (phase < 0 || phase == 2 || phase == 3)
+      rc = wide ? wide_launch(a, st, kWideDkv, sparse, half) : gen_launch_dkv(a, st, d, dtype, sparse);
     return rc;
   }
   if (phase < 0 || phase == 0) {

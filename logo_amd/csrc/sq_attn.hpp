@@ -439,6 +439,14 @@ int gen_launch_delta(const AttnArgs& a, hipStream_t st, int d, int dtype, bool s
 int gen_launch_dq(const AttnArgs& a, hipStream_t st, int d, int dtype, bool sparse);
 int gen_launch_dkv(const AttnArgs& a, hipStream_t st, int d, int dtype, bool sparse);
 
+// Head dim 256 in 16-bit types without a window (wide_attn.hip): whether it
+// serves a call (q and dO below 4 GB, as its gathered copies address them by 32
+// bits), its phases, and the workspace that lets its forward and dq split.
+enum { kWideFwd, kWideDelta, kWideDq, kWideDkv };
+bool wide_applies(const AttnArgs& a, int d, int dtype);
+size_t wide_workspace_bytes(int hq);
+int wide_launch(const AttnArgs& a, hipStream_t st, int phase, bool sparse, bool half);
+
 // Calls FN<D, SPARSE, WINDOW>(a, st) for the runtime (d, sparse, window).
 #define LOGO_DISPATCH(FN, a, st, d, sparse, window)                                                  \
   ((d) == 128 ? ((sparse) ? ((window) ? FN<128, true, true>(a, st) : FN<128, true, false>(a, st))   \

@@ -123,9 +123,13 @@ constexpr size_t kMaxCachedStreams = 16;
 
 at::Tensor split_workspace(const at::Tensor& q, const at::Tensor& cu, int dtype) {
   const char* env = std::getenv("LOGO_SQ_SPLIT");
-  const bool off = (env != nullptr && env[0] == '0') || generic_path(q, dtype);
-  const size_t bytes =
-      off ? 0 : logo_sq_workspace_bytes(q.size(0), (int)cu.numel() - 1, (int)q.size(1), (int)q.size(2));
+  size_t bytes = 0;
+  if (env == nullptr || env[0] != '0') {
+    if (!generic_path(q, dtype))
+      bytes = logo_sq_workspace_bytes(q.size(0), (int)cu.numel() - 1, (int)q.size(1), (int)q.size(2));
+    else if (dtype != LOGO_DTYPE_F32)
+      bytes = logo_sq_wide_workspace_bytes((int)q.size(1));
+  }
   if (bytes == 0) return at::empty({0}, q.options().dtype(at::kByte));
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   TORCH_CHECK(hipStreamIsCapturing(static_cast<hipStream_t>(sp()), &status) == hipSuccess,
