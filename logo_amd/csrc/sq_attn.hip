@@ -226,7 +226,8 @@ extern "C" int logo_sq_fwd(const void* q, const void* k, const void* v, void* o,
   a.ws_bytes = workspace ? workspace_bytes : 0;
   const bool sparse = q_idx != nullptr;
   const bool win = window >= 0;
-  if (wide_applies(a, d, dtype)) return wide_launch(a, as_stream(stream), kWideFwd, sparse, dtype == LOGO_DTYPE_F16);
+  if (f32_applies(a, d, dtype, sparse)) return f32_launch(a, as_stream(stream), kPhaseFwd, d);
+  if (wide_applies(a, d, dtype)) return wide_launch(a, as_stream(stream), kPhaseFwd, sparse, dtype == LOGO_DTYPE_F16);
   if (gen_applies(d, dtype)) return gen_launch_fwd(a, as_stream(stream), d, dtype, sparse);
   return sq_launch_fwd(a, as_stream(stream), d, sparse, win, dtype == LOGO_DTYPE_F16);
 }
@@ -272,17 +273,23 @@ static int bwd_entry(LOGO_BWD_PARAMS, int phase) {
   const bool half = dtype == LOGO_DTYPE_F16;
   hipStream_t st = as_stream(stream);
   if (generic) {  // these kernels read q and dO in place (no compacted copies)
-    const bool wide = wide_applies(a, d, dtype);
+    const bool f32 = f32_applies(a, d, dtype, sparse), wide = wide_applies(a, d, dtype);
+    auto run = [&](int ph) {
+      if (f32) return f32_launch(a, st, ph, d);
+      if (wide) return wide_launch(a, st, ph, sparse, half);
+      return ph == kPhaseDelta ? gen_launch_delta(a, st, d, dtype, sparse)
+             : ph == kPhaseDq  ? gen_launch_dq(a, st, d, dtype, sparse)
+                               : gen_launch_dkv(a, st, d, dtype, sparse);
+    };
     if (phase < 0 || phase == 0) {
-      rc = wide ? wide_launch(a, st, kWideDelta, sparse, half) : gen_launch_delta(a, st, d, dtype, sparse);
+      rc = run(kPhaseDelta);
       if (rc != LOGO_OK) return rc;
     }
     if (phase < 0 || phase == 1 || phase == 3) {
-      rc = wide ? wide_launch(a, st, kWideDq, sparse, half) : gen_launch_dq(a, st, d, dtype, sparse);
+      rc = run(kPhaseDq);
       if (rc != LOGO_OK) return rc;
     }
-    if (phase < 0 || phase == 2 || phase == 3)
-      rc = wide ? wide_launch(a, st, kWideDkv, sparse, half) : gen_launch_dkv(a, st, d, dtype, sparse);
+    if (phase < 0 || phase == 2 || phase == 3) rc = run(kPhaseDkv);
     return rc;
   }
   if (phase < 0 || phase == 0) {

@@ -439,10 +439,16 @@ int gen_launch_delta(const AttnArgs& a, hipStream_t st, int d, int dtype, bool s
 int gen_launch_dq(const AttnArgs& a, hipStream_t st, int d, int dtype, bool sparse);
 int gen_launch_dkv(const AttnArgs& a, hipStream_t st, int d, int dtype, bool sparse);
 
+// The phases of the kernel families below.
+enum { kPhaseFwd, kPhaseDelta, kPhaseDq, kPhaseDkv };
+
+// fp32 in sparse mode without a window (f32_attn.hip), q below 4 GB.
+bool f32_applies(const AttnArgs& a, int d, int dtype, bool sparse);
+int f32_launch(const AttnArgs& a, hipStream_t st, int phase, int d);
+
 // Head dim 256 in 16-bit types without a window (wide_attn.hip): whether it
 // serves a call (q and dO below 4 GB, as its gathered copies address them by 32
 // bits), its phases, and the workspace that lets its forward and dq split.
-enum { kWideFwd, kWideDelta, kWideDq, kWideDkv };
 bool wide_applies(const AttnArgs& a, int d, int dtype);
 size_t wide_workspace_bytes(int hq);
 int wide_launch(const AttnArgs& a, hipStream_t st, int phase, bool sparse, bool half);

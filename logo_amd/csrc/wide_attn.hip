@@ -877,8 +877,8 @@ int launch_rows(const AttnArgs& a_in, hipStream_t st, bool bwd) {
 
 template <typename EL, bool SPARSE>
 int launch(const AttnArgs& a, hipStream_t st, int phase) {
-  if (phase == kWideFwd || phase == kWideDq) return launch_rows<EL, SPARSE>(a, st, phase == kWideDq);
-  if (phase == kWideDelta) {
+  if (phase == kPhaseFwd || phase == kPhaseDq) return launch_rows<EL, SPARSE>(a, st, phase == kPhaseDq);
+  if (phase == kPhaseDelta) {
     hipLaunchKernelGGL((w256_delta_kernel<EL, SPARSE>), dim3((unsigned)((a.n + 15) / 16), a.hq), dim3(256), 0, st, a);
     LOGO_LAUNCH_CHECK("w256_delta_kernel");
     return LOGO_OK;
