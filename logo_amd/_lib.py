@@ -146,6 +146,10 @@ def set_launch_hook(hook):
     _launch_hook = hook
 
 
+def launch_hook_set() -> bool:
+    return _launch_hook is not None
+
+
 def launch(name: str, fn, *args):
     """Call C entry point ``fn`` (named ``name``), bracketed by the hook."""
     hook = _launch_hook
