@@ -13,6 +13,11 @@
 // from the group prefixes, then the tile prefixes (one lane of 32768 tokens
 // takes it in about 24 us, no faster than the three launches below, which
 // spread it over the GPU).
+// One lane of 4097 to 131072 tokens (16-byte aligned) takes one launch of
+// 1024-token workgroups that each read the whole mask (compact_flat): the mask
+// is a few KB and launches are about 5 us each (back to back in a graph, three
+// launches against one: 8192 tokens 18.7 / 4.6 us, 32768 20.1 / 6.1, 131072
+// 20.8 / 12.7; beyond, the n^2 / 1024 bytes read take over).
 // Everything else takes three launches, none of them synchronising with the
 // host:
 //   count    : per 4096-token chunk and lane, popcount of wave ballots
@@ -297,6 +302,91 @@ __global__ __launch_bounds__(256) void compact_finalize(const int32_t* __restric
   meta_tiles<256>(cu, nseq, n, sq, m, buf);
 }
 
+// Selected tokens among 16 mask bytes (any non-zero byte counts).
+__device__ __forceinline__ int count16(const u32x4 v) {
+  int c = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c += __popc((((v[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v[i]) & 0x80808080u);
+  return c;
+}
+
+// Selected tokens of sel[lo, hi), lo a multiple of 16 (sel 16-byte aligned).
+__device__ __forceinline__ int count_range(const uint8_t* __restrict__ sel, int64_t lo, int64_t hi) {
+  int c = 0;
+  for (; lo + 16 <= hi; lo += 16) c += count16(*reinterpret_cast<const u32x4*>(sel + lo));
+  for (; lo < hi; ++lo) c += sel[lo] != 0;
+  return c;
+}
+
+// The whole compaction of one lane in one launch (same outputs as count +
+// scatter + finalize).  Workgroup b < nchunk reads the mask once for the counts
+// before its kFlatChunk tokens and in all, then writes their entries; workgroup
+// nchunk writes the metadata.
+constexpr int kFlatChunk = 1024;
+constexpr int64_t kFlatMax = 131072;
+__global__ __launch_bounds__(256) void compact_flat(const uint8_t* __restrict__ sel, int64_t n,
+                                                    const int32_t* __restrict__ cu, int nseq, int nchunk,
+                                                    int64_t* __restrict__ qi, int32_t* __restrict__ ps,
+                                                    int32_t* __restrict__ meta) {
+  __shared__ int buf[4], red[4], base[256];
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  if ((int)blockIdx.x == nchunk) {
+    // thread t counts bytes [t per, (t + 1) per); cu_q[s] = what precedes the
+    // thread that holds token cu[s], and that thread's bytes before it
+    const int64_t per = (((n + 255) / 256) + 15) & ~(int64_t)15;
+    const int64_t lo = min(tid * per, n);
+    int sq;
+    base[tid] = block_exscan(count_range(sel, lo, min(lo + per, n)), buf, &sq);
+    __syncthreads();
+    for (int s = tid; s <= nseq; s += 256) {
+      const int64_t key = min((int64_t)cu[s], n);
+      const int owner = (int)min(key / per, (int64_t)255);
+      meta[kMetaHdr + s] = base[owner] + count_range(sel, owner * per, key);
+    }
+    __syncthreads();
+    meta_tiles<256>(cu, nseq, n, sq, meta, buf);
+    return;
+  }
+  const int64_t c0 = (int64_t)blockIdx.x * kFlatChunk;
+  uint64_t masks[4];
+  int cnt = 0;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    masks[s] = __ballot(sel_on(sel, n, 1, 0, c0 + w * 256 + s * 64 + l));
+    cnt += __popcll(masks[s]);
+  }
+  int part = 0, all = 0;
+  const int64_t n16 = n & ~(int64_t)15;
+  for (int64_t b = 16 * tid; b < n16; b += 16 * 256) {
+    const int v = count16(*reinterpret_cast<const u32x4*>(sel + b));
+    all += v;
+    if (b < c0) part += v;  // (c0 is a multiple of 16)
+  }
+  if (tid < (int)(n - n16)) all += sel[n16 + tid] != 0;
+  const int prefix = block_sum(part, red);
+  const int sq = block_sum(all, red);
+  if (l == 0) buf[w] = cnt;
+  __syncthreads();
+  int run = prefix;
+  for (int i = 0; i < w; ++i) run += buf[i];
+  const uint64_t below = (l == 0) ? 0ull : (~0ull >> (64 - l));
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const uint64_t m = masks[s];
+    const int rank = run + __popcll(m & below);  // selected tokens before t
+    const int64_t t = c0 + w * 256 + s * 64 + l;
+    if ((m >> l) & 1ull) {
+      const int sg = seg_of(cu, nseq, t);
+      qi[rank] = t;
+      ps[rank] = (int32_t)(t - cu[sg]);
+    } else if (t < n) {
+      qi[sq + (t - rank)] = 0;  // entries [Sq, N) are zero, as in compact_scatter
+      ps[sq + (t - rank)] = 0;
+    }
+    run += __popcll(m);
+  }
+}
+
 // prepare_chunk_indices for an arbitrary chunk size (parity helper).
 __global__ __launch_bounds__(256) void chunk_prefix_kernel(const int32_t* __restrict__ cu, int nseq,
                                                            int chunk, int32_t* __restrict__ prefix,
@@ -357,6 +447,13 @@ static int compact_launch(const uint8_t* selection, int64_t n_tokens, int lanes,
     hipLaunchKernelGGL(compact_small, dim3(lanes), dim3(kSmallThreads), 0, st, selection, n_tokens, lanes, cu, nseq,
                        q_idx, pos, meta);
     LOGO_LAUNCH_CHECK("compact_small");
+    return LOGO_OK;
+  }
+  if (lanes == 1 && n_tokens <= kFlatMax && reinterpret_cast<uintptr_t>(selection) % 16 == 0) {
+    const int nc = (int)((n_tokens + kFlatChunk - 1) / kFlatChunk);
+    hipLaunchKernelGGL(compact_flat, dim3(nc + 1), dim3(256), 0, st, selection, n_tokens, cu, nseq, nc, q_idx, pos,
+                       meta);
+    LOGO_LAUNCH_CHECK("compact_flat");
     return LOGO_OK;
   }
   const int nchunk = (int)((n_tokens + kChunk - 1) / kChunk);
