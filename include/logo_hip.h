@@ -148,10 +148,11 @@ int logo_q_start_blk(const int32_t* pos, const int32_t* cu_q, const int32_t* chu
  * dout, q_sel, do_sel, dq, dk, dv) holds that type.  d = 256 and fp32 run on
  * generic kernels (logo_sq_generic); the others on the tuned ones.
  * workspace / workspace_bytes (may be NULL / 0): device memory that lets the
- * forward and dq kernels (no window) cut the key range of each query tile
- * into pieces when a head has few tiles, so that a grid which would fill the
- * GPU once is not bound by its heaviest tile (the reference has no
- * counterpart: its grid is one program per chunk, :348 :413).  Its first
+ * forward and dq kernels (no window) cut the key range of each query tile,
+ * and dk/dv the query rows of each key block, into pieces when a head has few
+ * tiles, so that a grid which would fill the GPU once is not bound by its
+ * heaviest tile (the reference has no counterpart: its grid is one program per
+ * chunk, :348 :413).  Its first
  * bytes are arrival counters that must be zero when a call starts; every call
  * leaves them zero, so one zero-fill serves every later call.  Calls that
  * share a workspace must not overlap.  Too small (or NULL): no split.
@@ -163,8 +164,8 @@ int logo_sq_fwd(const void* q, const void* k, const void* v, void* o, float* lse
                 size_t workspace_bytes, void* stream);
 
 /*
- * Bytes of the workspace logo_sq_fwd and logo_sq_bwd_dq need to split tiles
- * on the current device (0: they never split for this shape), and how many
+ * Bytes of the workspace logo_sq_fwd, logo_sq_bwd_dq and logo_sq_bwd_dkv need
+ * to split tiles on the current device (0: they never split for this shape), and how many
  * of them, at its start, are the counters that must be zero.
  */
 size_t logo_sq_workspace_bytes(int64_t n_tokens, int nseq, int hq, int d);

@@ -202,7 +202,9 @@ extern "C" size_t logo_sq_workspace_bytes(int64_t n_tokens, int nseq, int hq, in
   const int cap_f = split_cap_for(hq, paired ? 1 : 2), cap_d = split_cap_for(hq, 2);
   const size_t fwd = cap_f >= 2 ? (size_t)hq * 2 * cap_f * fwd_part_floats(d, paired ? 8 : 4) : 0;
   const size_t dq = cap_d >= 2 ? (size_t)hq * 2 * cap_d * dq_part_floats(d) : 0;
-  const size_t part = std::max(fwd, dq) * sizeof(float);
+  // dk/dv: at most four pieces a CU for any number of kv heads
+  const size_t dkv = (size_t)4 * device_cus() * dkv_part_floats(d);
+  const size_t part = std::max({fwd, dq, dkv}) * sizeof(float);
   return part == 0 ? 0 : split_cnt_bytes() + part;
 }
 

@@ -39,7 +39,8 @@ struct AttnArgs {
   float scale;
   float scale_log2;
   int window;
-  // Key-range split of the fwd / dq tiles (no window): a tile is cut into up
+  // Key-range split of the fwd / dq tiles and row-range split of the dk/dv key
+  // blocks (no window; per kv head there): a tile is cut into up
   // to kMaxSplit pieces when its head has few tiles; each piece writes an fp32
   // partial to `part`, and the last piece of a tile to arrive (per-tile counter
   // in `cnt`, zero on entry, left zero) combines them.  split_cap: the pieces
@@ -91,12 +92,14 @@ inline size_t split_cnt_bytes() { return ((size_t)8 * device_cus() * sizeof(int)
 // [64] per wave), dq (2 waves x 2 row blocks x DT x 16 x 64).
 inline size_t fwd_part_floats(int d, int nw) { return (size_t)nw * ((size_t)(d / 32) * 16 * 64 + 64); }
 inline size_t dq_part_floats(int d) { return (size_t)2 * 2 * (d / 32) * 16 * 64; }
+// dk/dv: 4 waves x (dK, dV) x [d / 32][16][64]
+inline size_t dkv_part_floats(int d) { return (size_t)4 * 2 * (d / 32) * 16 * 64; }
 
 // Enables the split in `a` when its workspace holds the counters and
 // 2 split_cap pieces per head of `floats` each; otherwise split_cap = 0.
-inline void split_setup(AttnArgs& a, int wgs_per_cu, size_t floats) {
-  const int cap = split_cap_for(a.hq, wgs_per_cu);
-  const size_t need = split_cnt_bytes() + (size_t)a.hq * 2 * cap * floats * sizeof(float);
+inline void split_setup(AttnArgs& a, int heads, int wgs_per_cu, size_t floats) {
+  const int cap = split_cap_for(heads, wgs_per_cu);
+  const size_t need = split_cnt_bytes() + (size_t)heads * 2 * cap * floats * sizeof(float);
   if (cap >= 2 && a.ws != nullptr && a.ws_bytes >= need) {
     a.cnt = static_cast<int*>(a.ws);
     a.part = reinterpret_cast<float*>(static_cast<char*>(a.ws) + split_cnt_bytes());

@@ -4,6 +4,8 @@
 // through LDS, dK / dV of the whole group stored once in bf16.
 #include "sq_attn.hpp"
 
+#include <algorithm>
+
 namespace logo {
 
 // ---------------------------------------------------------------------------
@@ -16,6 +18,9 @@ namespace logo {
 // instruction offset, so the compiler keeps them in spare AGPRs.
 constexpr int kDkvRows = 128;
 constexpr int kDkvStages = 2;
+// Fewest steps a piece of a split key block takes: its partials cost about one
+// (128 KB at D = 128, written and read back).
+constexpr int kDkvMinSteps = 3;
 template <int D>
 constexpr int dkv_stage_bytes() { return 2 * kDkvRows * D * 2 + 3 * kDkvRows * 4; }
 
@@ -40,14 +45,43 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
   xcd_remap(blockIdx.x, a.h, rank, h);
   const int32_t* meta0 = a.meta;
   const int ntk = meta0[2];
-  if (rank >= ntk) return;
-  const int tile = rank;  // early key blocks (most queries) first
+  const int nper = WINDOW ? 1 : split_pieces(ntk, a.split_cap);
+  if (rank >= ntk * nper) return;
+  const int tile = rank / nper;  // early key blocks (most queries) first
+  const int piece = rank - tile * nper;
   const int32_t* cu_tk = meta0 + kMetaHdr + 2 * (a.nseq + 1);
   const int s = seg_of(cu_tk, a.nseq, tile);
   const int k0 = (tile - cu_tk[s]) * kBKV;
   const int bos = a.cu[s];
   const int seqlen = a.cu[s + 1] - bos;
   const int k_last = min(k0 + kBKV, seqlen) - 1;
+
+  // Row-range split of a key block (no window), where the kv heads have few
+  // key blocks (at most 3/4 of two workgroups a CU): the steps of all query
+  // heads of the group, one after the other, are cut into nsplit runs of at
+  // least kDkvMinSteps; this piece takes steps [st_lo, st_hi).  One workgroup a
+  // block left the GPU to its heaviest blocks (16 query, 4 kv heads of dim 64,
+  // 6001 tokens: 188 blocks of 1 to 48 steps on 256 CUs; forward + backward 215
+  // -> 183 us; 8 query, 2 kv heads, 4000 tokens, rows per head: 295 -> 186).
+  int nsplit = 1, st_lo = 0, st_hi = 0x7fffffff;
+  if (nper > 1) {
+    int total = 0;
+    for (int gg = 0; gg < a.g; ++gg) {
+      const int lane_sel = a.lanes > 1 ? h * a.g + gg : 0;
+      const int32_t* cu_q = a.meta + (int64_t)lane_sel * a.meta_stride + kMetaHdr;
+      const int lo = cu_q[s], hi = cu_q[s + 1];
+      const int r0 = SPARSE ? wave_lower_bound(row_view<SPARSE>(a, lane_sel, bos).ps, lo, hi, k0) : min(lo + k0, hi);
+      total += (hi - r0 + RS - 1) / RS;
+      if (a.lanes == 1) {  // every head has these rows
+        total *= a.g;
+        break;
+      }
+    }
+    nsplit = max(1, min(nper, total / kDkvMinSteps));
+    if (piece >= nsplit) return;
+    st_lo = total * piece / nsplit;
+    st_hi = total * (piece + 1) / nsplit;
+  }
 
   const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
   const int kw0 = k0 + 32 * wave;
@@ -102,8 +136,16 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
     auto lb_pos = [&](int lo, int hi, int x) {
       return SPARSE ? wave_lower_bound(rv.ps, lo, hi, x) : min(max(q_lo + x, lo), hi);
     };
-    const int rq0 = lb_pos(q_lo, q_hi, k0);
-    const int rq_end = WINDOW ? lb_pos(rq0, q_hi, k_last + W + 1) : q_hi;
+    int rq0 = lb_pos(q_lo, q_hi, k0);
+    int rq_end = WINDOW ? lb_pos(rq0, q_hi, k_last + W + 1) : q_hi;
+    if (nsplit > 1) {  // this piece's share of the head's steps
+      const int steps = (rq_end - rq0 + RS - 1) / RS;
+      const int lo = min(max(st_lo, 0), steps), hi = min(max(st_hi, 0), steps);
+      rq_end = min(rq_end, rq0 + RS * hi);
+      rq0 = min(rq_end, rq0 + RS * lo);
+      st_lo -= steps;
+      st_hi -= steps;
+    }
     // This wave's keys kw0 .. kw_last: rows before lb0 see none of them,
     // rows from lb1 on see all of them (causally), rows from lb2 on are past
     // the window of the last one.
@@ -425,6 +467,38 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
   }
 
   agpr_acc_drain();
+  if (nsplit > 1) {
+    // partial dK and dV of this piece as [wave][dK, dV][dt][item][lane]; the
+    // last piece of the key block to arrive adds all of them in piece order
+    constexpr int PW = 2 * DT * 16 * 64;  // floats per wave
+    float* const part0 = a.part + (int64_t)(h * 2 * a.split_cap + tile * nper) * 4 * PW + wave * PW + l;
+    {
+      float* pp = part0 + (int64_t)piece * 4 * PW;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          st_agent(pp + (dt * 16 + e) * 64, dkacc[dt][e]);
+          st_agent(pp + ((DT + dt) * 16 + e) * 64, dvacc[dt][e]);
+        }
+    }
+    if (!split_arrive(a.cnt + h * 2 * a.split_cap + tile, nsplit, reinterpret_cast<int*>(smem_b))) return;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      f32x16 sk = f32x16{}, sv = f32x16{};
+      for (int pc = 0; pc < nsplit; ++pc) {
+        const float* pp = part0 + (int64_t)pc * 4 * PW;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          sk[e] += ld_agent(pp + (dt * 16 + e) * 64);
+          sv[e] += ld_agent(pp + ((DT + dt) * 16 + e) * 64);
+        }
+      }
+      dkacc[dt] = sk;
+      dvacc[dt] = sv;
+    }
+    __syncthreads();  // the flag is read: LDS is free again
+  }
   // dK and dV leave through LDS (free after the last step's barrier) as whole
   // rows: each wave writes its 32 keys' rows (8-byte pieces into swizzled
   // chunks), then 16 lanes store one row's D * 2 bytes together.  Stored from
@@ -470,11 +544,16 @@ template <int D>
 constexpr size_t dkv_smem() { return (size_t)kDkvStages * dkv_stage_bytes<D>(); }
 
 template <typename EL, int D, bool SPARSE, bool WINDOW>
-static int launch_dkv(const AttnArgs& a, hipStream_t st) {
+static int launch_dkv(const AttnArgs& a_in, hipStream_t st) {
+  AttnArgs a = a_in;
   const int64_t ntmax = (a.n + kBKV - 1) / kBKV + a.nseq;
+  if (WINDOW) a.split_cap = 0;
+  else split_setup(a, a.h, 1, dkv_part_floats(D));
+  const int64_t nblk = std::max<int64_t>(ntmax, 2 * a.split_cap) * a.h;
+  LOGO_REQUIRE(nblk < ((int64_t)1 << 31), "grid too large");
   auto kern = sq_dkv_kernel<EL, D, SPARSE, WINDOW>;
   LOGO_HIP_CHECK(allow_smem(kern, dkv_smem<D>()));
-  hipLaunchKernelGGL(kern, dim3((unsigned)(ntmax * a.h)), dim3(256), dkv_smem<D>(), st, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(256), dkv_smem<D>(), st, a);
   LOGO_LAUNCH_CHECK("sq_dkv_kernel");
   return LOGO_OK;
 }

@@ -204,7 +204,7 @@ struct Bwd {
     F fn = phase == 0 ? &logo_sq_bwd_delta : phase == 1 ? &logo_sq_bwd_dq : phase == 2 ? &logo_sq_bwd_dkv
                                                                                   : &logo_sq_bwd_dqkv;
     auto p = [](at::Tensor* t) -> void* { return t && t->numel() ? t->data_ptr() : nullptr; };
-    at::Tensor ws = (phase == 1 || phase == 3) && window < 0 ? split_workspace(q, cu, dtype)
+    at::Tensor ws = phase >= 1 && window < 0 ? split_workspace(q, cu, dtype)
                                                             : at::empty({0}, q.options().dtype(at::kByte));
     return fn(cptr(q), cptr(k), cptr(v), cptr(o), cptr(dout), lse.data_ptr<float>(),
               static_cast<float*>(p(delta)), p(q_sel), p(do_sel), p(dq), p(dk), p(dv), opt_ptr<int64_t>(q_idx),
