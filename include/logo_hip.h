@@ -412,6 +412,38 @@ int logo_head_linear_grad_acc(const void* dy, int64_t lddy, const void* w, const
                               int64_t lddx, int64_t n_tokens, int heads, int d, int dtype, void* stream);
 
 /*
+ * The global maps of up to three contiguous [n_tokens, h_i, d] tensors (d = 64
+ * or 128) and the rotary embedding of inputs and outputs in one launch
+ * (logo/layers/logo.py:86-94, logo/modules/rotary.py:81-106), the same bits as
+ * logo_head_linear and logo_rope one after the other:
+ *   xr_i = rope(x_i), y_i = rope(x_i W_i)   where xr_i is not null (it may be x_i),
+ *   y_i = x_i W_i                           where it is.
+ * w_i [h_i, d, d]; cos / sin [n_tokens, d] (may be null if no xr_i is given).
+ * Unused x_i are null.  All pointers 16-byte aligned.
+ */
+int logo_global_maps(const void* x0, const void* w0, void* xr0, void* y0, int h0, const void* x1, const void* w1,
+                     void* xr1, void* y1, int h1, const void* x2, const void* w2, void* xr2, void* y2, int h2,
+                     const void* cos, const void* sin, int64_t n_tokens, int d, int dtype, void* stream);
+
+/*
+ * Backward of logo_global_maps (d = 128): with da_i the gradient of xr_i (of x_i
+ * as a direct output where rope_i is 0) and dg_i that of y_i, each [n_tokens,
+ * h_i, d] and contiguous,
+ *   dg' = rope_i ? rope^T(dg_i) : dg_i, da' likewise,
+ *   dx_i = bf16(dg' W_i^T) + da'   (rows of stride lddx, below 2^23),
+ *   dw_i = x_i^T dg'               (skipped where dw_i is null),
+ * the same bits as logo_rope (inverse), logo_head_linear_grad_acc and
+ * logo_head_linear_dw one after the other.  workspace:
+ * logo_head_linear_dw_workspace_bytes(n_tokens, h0 + h1 + h2, d) bytes (may be
+ * null if no dw_i is given).
+ */
+int logo_global_maps_bwd(const void* x0, const void* w0, const void* da0, const void* dg0, void* dx0, void* dw0,
+                         int h0, int rope0, const void* x1, const void* w1, const void* da1, const void* dg1,
+                         void* dx1, void* dw1, int h1, int rope1, const void* x2, const void* w2, const void* da2,
+                         const void* dg2, void* dx2, void* dw2, int h2, int rope2, const void* cos, const void* sin,
+                         int64_t lddx, void* workspace, int64_t n_tokens, int d, int dtype, void* stream);
+
+/*
  * Residual add + RMSNorm of the decoder: s_out = r + x (bf16, as the eager
  * add rounds) and y = RMSNorm(s_out) with weight w (as logo_rmsnorm), rows of
  * cols bf16 (a multiple of 8, at most 4096): the residual adds and the

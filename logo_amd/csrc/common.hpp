@@ -317,8 +317,10 @@ struct TileBufDma {
   __device__ __forceinline__ static int wave_s() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
   // Rows row0 .. row0 + 63, all valid.
-  __device__ __forceinline__ void issue(bf16* tile, const bf16* row0) const {
-    const auto r = rsrc(row0);
+  __device__ __forceinline__ void issue(bf16* tile, const bf16* row0) const { issue(tile, rsrc(row0)); }
+
+  // The rows of a descriptor of the caller's, whose extent may end earlier.
+  __device__ __forceinline__ void issue(bf16* tile, __amdgpu_buffer_rsrc_t r) const {
     const int wave = wave_s();
 #pragma unroll
     for (int b = 0; b < BLOCKS; ++b) {
@@ -436,6 +438,31 @@ __device__ __forceinline__ float group_sum(float v) {
 }
 
 __device__ __forceinline__ float bfr(float x) { return (float)(bf16)x; }
+
+// Rotary embedding (INV: its transpose) of a pair of chunks, x1 of the first
+// and x2 of the second half of a row, in place; every product and sum rounds
+// as its own eager bf16 op (no fma contraction).
+template <bool INV>
+__device__ __forceinline__ void rope_chunk(bf16x8& x1, bf16x8& x2, const bf16x8 c1, const bf16x8 c2, const bf16x8 s1,
+                                           const bf16x8 s2) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float u = (float)x1[e], v = (float)x2[e];
+    const float a1 = bfr(u * (float)c1[e]), a2 = bfr(v * (float)c2[e]);
+    if constexpr (!INV) {
+      // first half:  x1 * cos1 + (-x2) * sin1;  second half: x2 * cos2 + x1 * sin2
+      const float b1 = bfr(-v * (float)s1[e]), b2 = bfr(u * (float)s2[e]);
+      x1[e] = (bf16)(a1 + b1);
+      x2[e] = (bf16)(a2 + b2);
+    } else {
+      // transpose of the rotation: x1 * cos1 + x2 * sin2;  x2 * cos2 - x1 * sin1
+      const float b1 = bfr(v * (float)s2[e]), b2 = -bfr(u * (float)s1[e]);
+      x1[e] = (bf16)(a1 + b1);
+      x2[e] = (bf16)(a2 + b2);
+    }
+  }
+}
 
 // Fused attention epilogue of one (token, head) row of D elements, held by D/8
 // consecutive lanes (lane c owns elements 8c..8c+7), with the eager bf16

@@ -66,27 +66,8 @@ __global__ __launch_bounds__(256) void rope_kernel(const RopeArgs a, int64_t per
   const bf16x8 c2 = *reinterpret_cast<const bf16x8*>(a.cos + tok * D + D / 2 + 8 * c);
   const bf16x8 s1 = *reinterpret_cast<const bf16x8*>(a.sin + tok * D + 8 * c);
   const bf16x8 s2 = *reinterpret_cast<const bf16x8*>(a.sin + tok * D + D / 2 + 8 * c);
-  bf16x8 y1, y2;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    if constexpr (!INV) {
-      // first half:  x1 * cos1 + (-x2) * sin1;  second half: x2 * cos2 + x1 * sin2
-      const float a1 = bfr_g((float)x1[e] * (float)c1[e]);
-      const float b1 = bfr_g(-(float)x2[e] * (float)s1[e]);
-      const float a2 = bfr_g((float)x2[e] * (float)c2[e]);
-      const float b2 = bfr_g((float)x1[e] * (float)s2[e]);
-      y1[e] = (bf16)(a1 + b1);
-      y2[e] = (bf16)(a2 + b2);
-    } else {
-      // transpose of the rotation: x1 * cos1 + x2 * sin2;  x2 * cos2 - x1 * sin1
-      const float a1 = bfr_g((float)x1[e] * (float)c1[e]);
-      const float b1 = bfr_g((float)x2[e] * (float)s2[e]);
-      const float a2 = bfr_g((float)x2[e] * (float)c2[e]);
-      const float b2 = -bfr_g((float)x1[e] * (float)s1[e]);
-      y1[e] = (bf16)(a1 + b1);
-      y2[e] = (bf16)(a2 + b2);
-    }
-  }
+  bf16x8 y1 = x1, y2 = x2;
+  rope_chunk<INV>(y1, y2, c1, c2, s1, s2);
   st_nt(reinterpret_cast<bf16x8*>(yr + 8 * c), y1);
   st_nt(reinterpret_cast<bf16x8*>(yr + D / 2 + 8 * c), y2);
 }

@@ -29,7 +29,8 @@ import torch.nn.functional as F
 
 from .ops.decode import LogoKVCache, decode_attn, decode_attn_fused, decode_qkv
 from .ops.epilogue import logo_epilogue
-from .ops.glue import attn_inputs, dec_linear, dec_linear_ok, head_linear, head_proj, rms_norm, rope, rope_apply_
+from .ops.glue import (attn_inputs, dec_linear, dec_linear_ok, global_maps_, global_maps_ok, head_linear, head_proj,
+                       rms_norm, rope, rope_apply_)
 from .ops.sq_attn import dense_causal_attn, sq_full_attn, swa_attn
 
 __all__ = ["LoGoConfig", "LoGoAttention", "Attention", "RMSNorm", "rope_cos_sin", "apply_rope", "position_ids_for"]
@@ -348,6 +349,15 @@ class LoGoAttention(nn.Module):
         return (self.head_dim == 128 and B * T > 64
                 and all(t.is_cuda and t.dtype == torch.bfloat16 for t in (hidden_states, *ws)))
 
+    def _maps_fused_ok(self, q, k, v, cos, sin) -> bool:
+        """Prefill-size bf16 calls of the linear_proj form without gradients
+        take the global maps and RoPE as one launch (up to 64 tokens the maps
+        are a launch of their own, see ``_global_qkv``)."""
+        if self.global_qk_param != "linear_proj" or q.shape[0] * q.shape[1] <= 64:
+            return False
+        ws = (self.q_global_proj, self.k_global_proj, self.v_global_proj)
+        return _fused_ok(q, k, v, cos, sin, *ws) and global_maps_ok(q, k, v, ws, cos, sin)
+
     def _fuse(self, local, glob, gate):
         """Context norms + gate mask + fusion; ``local/glob [B, T, H, D]``."""
         if self.use_context_norm:
@@ -446,11 +456,15 @@ class LoGoAttention(nn.Module):
             q = self.q_proj(hidden_states).view(B, T, H, D)
             k = self.k_proj(hidden_states).view(B, T, HK, D)
             v = self.v_proj(hidden_states).view(B, T, HK, D)
-            gq, gk, gv = self._global_qkv(q, k, v)
-            gate = torch.sigmoid(self.gate_proj(hidden_states))  # [B, T, 1]
             if cos is None:
                 cos, sin = cs(q.dtype)
-            q, k, gq, gk = _rope_all((q, k, gq, gk), cos, sin)
+            if self._maps_fused_ok(q, k, v, cos, sin):
+                q, k, v, gq, gk, gv = global_maps_(q, k, v, (self.q_global_proj, self.k_global_proj,
+                                                             self.v_global_proj), cos, sin)
+            else:
+                gq, gk, gv = self._global_qkv(q, k, v)
+                q, k, gq, gk = _rope_all((q, k, gq, gk), cos, sin)
+            gate = torch.sigmoid(self.gate_proj(hidden_states))  # [B, T, 1]
 
         if past_key_value is not None and T == 1:
             out = self._decode(q, k, v, gq, gk, gv, gate, past_key_value)

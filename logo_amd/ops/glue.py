@@ -15,8 +15,8 @@ import torch.nn.functional as F
 from .. import _lib
 
 __all__ = ["rope_apply_", "rope", "RopeFunction", "rms_norm", "head_proj", "add_rms_norm", "silu_mul",
-           "dec_linear", "dec_linear_ok", "head_linear", "HeadLinearFunction", "head_linear_grad_acc", "attn_inputs",
-           "AttnInputsFunction"]
+           "dec_linear", "dec_linear_ok", "head_linear", "HeadLinearFunction", "head_linear_grad_acc",
+           "global_maps_", "global_maps_ok", "attn_inputs", "AttnInputsFunction"]
 
 
 def _rope_checked(tensors, cos, sin, what):
@@ -296,6 +296,52 @@ def head_linear_grad_acc(dy, w, add, out):
     return out
 
 
+def _global_maps_ok(ts) -> bool:
+    """Whether tensors can be operands of the fused global maps as they are:
+    contiguous and starting at a multiple of 16 bytes."""
+    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in ts)
+
+
+def _global_maps_launch(xs, ws, cos, sin, inplace: bool):
+    """``(rope(q), rope(k), v, rope(q Wq), rope(k Wk), v Wv)`` of contiguous
+    bf16 ``xs = (q, k, v)`` (rotated in place with ``inplace``)."""
+    D = xs[0].shape[-1]
+    n = xs[0][..., 0, 0].numel()
+    ys = [torch.empty_like(x) for x in xs]
+    rs = [x if inplace else torch.empty_like(x) for x in xs[:2]]
+    args = []
+    for x, w, r, y in zip(xs, ws, (*rs, None), ys):
+        args += [_lib.ptr(x), _lib.ptr(w), _lib.ptr(r), _lib.ptr(y), x.shape[-2]]
+    lib = _lib.lib()
+    _lib.launch("logo_global_maps", lib.logo_global_maps, *args, _lib.ptr(cos), _lib.ptr(sin), n, D, _lib.DTYPE_BF16,
+                _lib.stream_of(xs[0]))
+    return (*rs, xs[2], *ys)
+
+
+def global_maps_ok(q, k, v, ws, cos, sin) -> bool:
+    """Whether ``global_maps_`` takes these operands: bf16 ROCm tensors, all
+    contiguous and aligned, head dim 64 or 128, square per-head maps."""
+    D, lead = q.shape[-1], q.shape[:-2]
+    n = q[..., 0, 0].numel()
+    return (D in (64, 128) and 0 < n < 1 << 31
+            and all(t.is_cuda and t.dtype == torch.bfloat16 for t in (q, k, v, *ws, cos, sin))
+            and all(x.shape[:-2] == lead and x.shape[-1] == D and x.shape[-2] <= 4096
+                    and tuple(w.shape) == (x.shape[-2], D, D) for x, w in zip((q, k, v), ws))
+            and cos.numel() == sin.numel() == n * D and _global_maps_ok((q, k, v, *ws, cos, sin)))
+
+
+def global_maps_(q, k, v, ws, cos, sin):
+    """The attention inputs of a layer from its projections ``q, k, v [..., T,
+    H_i, D]`` without gradients, one launch: rotates q and k in place with
+    ``cos/sin [..., T, D]`` and returns them with v and the per-head maps
+    ``(q, k, v, rope(q Wq), rope(k Wk), v Wv)``, the maps taken of the inputs
+    before their rotation."""
+    if not global_maps_ok(q, k, v, ws, cos, sin):
+        raise ValueError("global_maps_ takes contiguous bf16 [..., T, H, D] ROCm tensors and square per-head maps")
+    _lib.require_gpu(q, k, v, *ws, cos, sin)
+    return _global_maps_launch((q, k, v), ws, cos, sin, inplace=True)
+
+
 class HeadLinearFunction(torch.autograd.Function):
     """``y[..., h, :] = x[..., h, :] @ w[h]`` with its gradients, every pass on
     the ``[..., H, D]`` layout in place (no head-major copies)."""
@@ -335,15 +381,15 @@ class AttnInputsFunction(torch.autograd.Function):
 
         q, k, v    = h Wq^T + bq, h Wk^T + bk, h Wv^T + bv   (hipBLASLt GEMMs)
         logit      = h wg^T + bg                            (the gate, before its sigmoid)
-        gq, gk, gv = per-head maps of q, k, v               (head_linear)
-        returns      rope(q), rope(k), v, rope(gq), rope(gk), gv, logit   (one RoPE launch)
+        gq, gk, gv = per-head maps of q, k, v
+        returns      rope(q), rope(k), v, rope(gq), rope(gk), gv, logit   (one launch with the maps)
 
-    The forward launches exactly the ops of the unfused chain.  The backward
+    The forward gives the bits of the unfused chain.  The backward
     differs in where sums happen, not in the products: q, k and v each feed
     the local branch and their global map, and h feeds four projections, so
-    autograd would add gradient pairs in separate passes.  Here the RoPE
-    backward runs once over the four rotated gradients, the global maps' input
-    gradients are written by ``head_linear_grad_acc`` together with the local
+    autograd would add gradient pairs in separate passes.  Here one launch
+    rotates the four gradients back, takes the maps' weight gradients and
+    writes their input gradients together with the local
     gradients (the same bf16 values as the separate add) straight into one
     ``[N, (H + 2 HK) D + 8]`` buffer whose last columns hold the gate logit's
     gradient and seven zeros, and dh is one GEMM of that buffer with the
@@ -362,30 +408,39 @@ class AttnInputsFunction(torch.autograd.Function):
         v = F.linear(h, wv, bv).view(B, T, kv_heads, D)
         logit = F.linear(h, wg, bg)
         gws = [w.contiguous() for w in (gwq, gwk, gwv)]
-        gq, gk, gv = (_head_linear_launch(x, w, False) for x, w in zip((q, k, v), gws))
-        cos, sin, n, _ = _rope_checked([q, k, gq, gk], cos, sin, "attn_inputs")
-        qr, kr, gqr, gkr = _rope_launch([q, k, gq, gk], cos, sin, n, D, inverse=False)
+        cos, sin, n, _ = _rope_checked([q, k], cos, sin, "attn_inputs")
+        ops = [_aligned16(t) for t in (q, k, v, *gws, cos, sin)]
+        qr, kr, _, gqr, gkr, gv = _global_maps_launch(ops[:3], ops[3:6], *ops[6:], inplace=False)
         ctx.save_for_backward(h, wq, wk, wv, wg, q, k, v, *gws, cos, sin)
         ctx.dims = (B, T, C, heads, kv_heads, D, n)
         return qr, kr, v, gqr, gkr, gv, logit
 
     @staticmethod
     def backward(ctx, dqr, dkr, dv, dgqr, dgkr, dgv, dlogit):
-        h, wq, wk, wv, wg, q, k, v, gwq, gwk, gwv, cos, sin = ctx.saved_tensors
+        h, wq, wk, wv, wg, *saved = ctx.saved_tensors
+        q, k, v, gwq, gwk, gwv, cos, sin = (_aligned16(t) for t in saved)
         B, T, C, H, HK, D, n = ctx.dims
         need = ctx.needs_input_grad
-        bf = lambda g: g.to(torch.bfloat16).contiguous()  # noqa: E731
-        dqr, dkr, dv, dgqr, dgkr, dgv = (bf(g) for g in (dqr, dkr, dv, dgqr, dgkr, dgv))
-        dqa, dka, dgq, dgk = _rope_launch([dqr, dkr, dgqr, dgkr], cos, sin, n, D, inverse=True)
+        bf = lambda g: _aligned16(g.to(torch.bfloat16))  # noqa: E731
+        das, dgs = [bf(g) for g in (dqr, dkr, dv)], [bf(g) for g in (dgqr, dgkr, dgv)]
         cols = (H * D, HK * D, HK * D, 8)
         dy = torch.empty(n, sum(cols), dtype=torch.bfloat16, device=h.device)
         outs = dy.split(cols, dim=1)
-        for g, w, a, o, nh in zip((dgq, dgk, dgv), (gwq, gwk, gwv), (dqa, dka, dv), outs, (H, HK, HK)):
-            head_linear_grad_acc(g.view(n, nh, D), w, a.view(n, nh, D), o.view(n, nh, D))
+        lib = _lib.lib()
+        dgw, ws = [None] * 3, None
+        if any(need[9:12]):
+            ws = torch.empty((lib.logo_head_linear_dw_workspace_bytes(n, H + 2 * HK, D) + 3) // 4,
+                             dtype=torch.float32, device=h.device)
+            dgw = [torch.empty(nh, D, D, dtype=torch.bfloat16, device=h.device) if need[9 + i] else None
+                   for i, nh in enumerate((H, HK, HK))]
+        args = []
+        for i, (x, w, nh) in enumerate(((q, gwq, H), (k, gwk, HK), (v, gwv, HK))):
+            args += [_lib.ptr(x), _lib.ptr(w), _lib.ptr(das[i]), _lib.ptr(dgs[i]), _lib.ptr(outs[i]),
+                     _lib.ptr(dgw[i]), nh, int(i < 2)]
+        _lib.launch("logo_global_maps_bwd", lib.logo_global_maps_bwd, *args, _lib.ptr(cos), _lib.ptr(sin),
+                    dy.stride(0), _lib.ptr(ws), n, D, _lib.DTYPE_BF16, _lib.stream_of(dy))
         outs[3].zero_()
         outs[3][:, 0].copy_(dlogit.reshape(n))
-        dgw = [_head_linear_dw(x, g).to(w.dtype) if need[9 + i] else None
-               for i, (x, g, w) in enumerate(zip((q, k, v), (dgq, dgk, dgv), (gwq, gwk, gwv)))]
         h2 = h.reshape(n, C)
         dh = None
         if need[0]:
