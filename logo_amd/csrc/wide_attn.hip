@@ -14,7 +14,7 @@
 // registers hold no second row block), 1 KB per 32 cycles and SIMD: all of the
 // LDS bandwidth at the MFMA peak, so about half of that peak is the aim.
 // Measured at T = 8192, 16 heads, a quarter of the rows, forward + backward:
-// 876 us, 1833 on the generic kernels (16 rows or keys a wave on 16x16 MFMAs,
+// 822 us, 1834 on the generic kernels (16 rows or keys a wave on 16x16 MFMAs,
 // one LDS operand read per half as many FLOPs, no pipelining); 4001 tokens, 4
 // heads, forward only with split key ranges: 70 against 227 us; a few hundred
 // tokens are bound by the launches either way.
@@ -645,17 +645,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       const auto ro = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a.dout + (int64_t)hq * D), (short)0, -1,
                                                         kBufRsrcWord3);
       // token of row i of step t, loaded a step ahead of the copy that uses it
-      auto load_tok = [&](int t) { return (int)rv.token(min(rq0 + RS * t + i, rq_end - 1)); };
+      // (the low half of the index: as a 64-bit load, whose dead half's register
+      // is used again, it had every step wait for its own copies: 42% of the
+      // wave time was waiting, forward + backward took 876 us in place of 822 us
+      // at T = 8192, 16 heads, a quarter of the rows)
+      auto load_tok = [&](int t) {
+        const int r = min(rq0 + RS * t + i, rq_end - 1);
+        return SPARSE ? reinterpret_cast<const int*>(rv.qi)[2 * r] : r;
+      };
       // a statistic of row i of step t: lse in wave 0, delta in wave 1, the
       // position in wave 2 (rows past the end repeat the last one, at position
-      // -1: they see no key)
-      auto load_stat = [&](int t) {
-        const int rr = rq0 + RS * t + i, rc = min(rr, rq_end - 1);
-        if (wave == 0) return __float_as_int(lse_h[rc]);
-        if (wave == 1) return __float_as_int(delta_h[rc]);
-        return rr < rq_end ? rv.posn(rr) : -1;
-      };
+      // -1: they see no key); one load on every path, for the count at the end
+      // of the step
+      const int* const stat_src = wave == 1                  ? reinterpret_cast<const int*>(delta_h)
+                                  : (SPARSE && wave >= 2) ? reinterpret_cast<const int*>(rv.ps)
+                                                          : reinterpret_cast<const int*>(lse_h);
+      auto load_stat = [&](int t) { return stat_src[min(rq0 + RS * t + i, rq_end - 1)]; };
       auto store_stat = [&](int t, int v) {
+        const int rr = rq0 + RS * t + i;
+        if (wave == 2) v = rr >= rq_end ? -1 : SPARSE ? v : rv.posn(rr);
         if (wave < 3 && l < RS) reinterpret_cast<int*>(stat(t))[RS * wave + l] = v;
       };
       auto load_tile = [&](int t, int tok) {  // wave w copies rows 8 w .. 8 w + 7, two a load
@@ -784,27 +792,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         });
         __builtin_amdgcn_sched_barrier(0);
       };
-      int tok = load_tok(0), tok1 = load_tok(1), st0 = load_stat(0), st1 = load_stat(1);
-      load_tile(0, tok);
-      store_stat(0, st0);
-      tok = load_tok(2);
-      if (nt > 1) load_tile(1, tok1);
-      store_stat(1, st1);
-      step_end(nt > 1);
+      {
+        const int tok0 = load_tok(0), tok1 = load_tok(1), st0 = load_stat(0), st1 = load_stat(1);
+        load_tile(0, tok0);
+        load_tile(1, tok1);
+        store_stat(0, st0);
+        store_stat(1, st1);
+      }
+      int tok[2] = {load_tok(2), load_tok(3)}, stn[2] = {0, load_stat(2)};
+      step_end(false);
+      // landed here: pending at the loop's entry, each turn would wait for all
+      asm volatile("" : "+v"(tok[0]), "+v"(tok[1]), "+v"(stn[1]));
       using T_ = std::true_type;
       using F_ = std::false_type;
       // step t; the last (t = nt) finishes step nt - 1 (what it forms of step nt
       // comes from old tiles and is never used)
-      int stn = 0;
+      // Step t copies the rows of step t + 2 and loads the statistics of t + 3 and
+      // the tokens of t + 4 (past the end: of the last row, into free slots), so
+      // that a step waits for nothing that it issued itself: at its end the copies
+      // of step t - 1 have landed, behind which 12 operations were issued (10
+      // without token indices to load).
       auto step = [&](auto par_tag, int t) {
-        const bool newest = t + 2 < nt;
-        if (newest) {
-          stn = load_stat(t + 2);
-          const int tk = tok;
-          tok = load_tok(t + 3);
-          load_tile(t + 2, tk);
-        }
-        const bool dox = t >= t_lo && t < nt, doy = t - 1 >= t_lo && t >= 1;
+        constexpr int PAR = decltype(par_tag)::value;
+        asm volatile("" ::: "memory");
+        load_tile(t + 2, tok[PAR]);
+        asm volatile("" ::: "memory");
+        stn[PAR] = load_stat(t + 3);
+        tok[PAR] = load_tok(t + 4);
+        asm volatile("" ::: "memory");
+        const bool dox = t >= t_lo && t < nt, doy = t - 1 >= t_lo && t >= 1 && t <= nt;
         if constexpr (!ROLE_B) {
           const bool mask = rq0 + RS * t < lb1 || rq0 + RS * (t + 1) > rq_end;
           if (doy) {
@@ -817,12 +833,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
           if (doy) step_b(par_tag, T_{}, t);
           else if (dox) step_b(par_tag, F_{}, t);
         }
-        if (newest) store_stat(t + 2, stn);
-        step_end(newest);
+        store_stat(t + 2, stn[PAR ^ 1]);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(SPARSE ? 12 : 10) : "memory");
       };
       for (int t = 0; t <= nt; t += 2) {
         step(BufTag<0>{}, t);
-        if (t + 1 <= nt) step(BufTag<1>{}, t + 1);
+        step(BufTag<1>{}, t + 1);  // (may be past the last: on every path, for the waits' counts)
         agpr_acc_drain();  // the accumulators may be read next
       }
     }
