@@ -145,8 +145,10 @@ int logo_q_start_blk(const int32_t* pos, const int32_t* cu_q, const int32_t* chu
  * dtype: LOGO_DTYPE_BF16; LOGO_DTYPE_F16 or LOGO_DTYPE_F32 in sparse mode
  * without a window (the reference's dots run in the input dtype, :80 :93-99
  * :108).  Every element tensor of the call (q, k, v, o, and for the backward
- * dout, q_sel, do_sel, dq, dk, dv) holds that type.  d = 256 and fp32 run on
- * generic kernels (logo_sq_generic); the others on the tuned ones.
+ * dout, q_sel, do_sel, dq, dk, dv) holds that type.  d = 64 and 128 in
+ * 16-bit types run on the tuned kernels; d = 256 and fp32 (logo_sq_generic) on
+ * kernels of their own without a window and with q below 4 GB, on the generic
+ * ones else.
  * workspace / workspace_bytes (may be NULL / 0): device memory that lets the
  * forward and dq kernels (no window) cut the key range of each query tile,
  * and dk/dv the query rows of each key block, into pieces when a head has few
@@ -179,11 +181,12 @@ size_t logo_sq_workspace_counter_bytes(void);
 size_t logo_sq_wide_workspace_bytes(int hq);
 
 /*
- * 1 when calls with head dim d and element type dtype run on the generic
- * attention kernels (d = 256, or LOGO_DTYPE_F32), 0 for the tuned ones (no
- * counterpart in the reference, whose Triton kernels take every size).  The
- * generic kernels take no split workspace, and their sparse backward reads q
- * and dout in place: q_sel and do_sel may be NULL.
+ * 1 when the sparse backward of head dim d and element type dtype reads q and
+ * dout in place, so that q_sel and do_sel may be NULL (d = 256, or
+ * LOGO_DTYPE_F32: the wide, fp32 and generic kernels), 0 for the tuned kernels
+ * (no counterpart in the reference, whose Triton kernels take every size).  Of
+ * the former only the 16-bit d = 256 kernels without a window split, with the
+ * workspace of logo_sq_wide_workspace_bytes.
  */
 int logo_sq_generic(int d, int dtype);
 

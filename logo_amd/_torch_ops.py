@@ -91,7 +91,7 @@ def _register_fakes():
 
 def generic_kernels(d: int, dtype: torch.dtype) -> bool:
     """Whether head dim ``d`` and element type ``dtype`` run on the library's
-    generic attention kernels (``logo_sq_generic``: d = 256 or fp32)."""
+    kernels that read q and dO in place (``logo_sq_generic``: d = 256 or fp32)."""
     code = {torch.float16: _lib.DTYPE_F16, torch.float32: _lib.DTYPE_F32}.get(dtype, _lib.DTYPE_BF16)
     return bool(_lib.lib().logo_sq_generic(int(d), code))
 

@@ -4,7 +4,8 @@
 //     zero-padded by the caller) with a sliding window, or with q above 4 GB
 //     (wide_attn.hip takes the others): the reference takes any K <= 256 in one
 //     block (logo/ops/selected_full_attn.py:344, logo/ops/common.py:127-168);
-//   * fp32 q, k, v on the query-sparse path, computed in fp32 throughout:
+//   * fp32 q, k, v on the query-sparse path with q above 4 GB (f32_attn.hip
+//     takes the others), computed in fp32 throughout:
 //     the reference's dots run in the input dtype, P kept in fp32 for PV
 //     (logo/ops/selected_full_attn.py:93-99) and the output in v's dtype
 //     (:349).

@@ -25,7 +25,7 @@ _custom_bwd = functools.partial(torch.amp.custom_bwd, device_type="cuda")
 
 
 # Head dims the gfx950 kernels are compiled for: 64 and 128 on the tuned
-# kernels, 256 on the generic ones.  A call with other K, V <= 256 (V != K
+# kernels, 256 on the wide ones.  A call with other K, V <= 256 (V != K
 # included, as the reference allows: its V is a separate constexpr and K fits
 # one block of <= 256, logo/ops/selected_full_attn.py:341-351, :344) runs on
 # the next compiled dim with q, k and v zero-padded: zero columns add nothing
