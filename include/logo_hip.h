@@ -322,6 +322,17 @@ int logo_cache_append(const void* k_new, const void* v_new, void* k_cache, void*
                       int dtype, void* stream);
 
 /*
+ * Store a prompt's keys and values of one layer, rows [B, T, H, D] (16-bit, d =
+ * 64 or 128, T <= t_cap), into an empty cache (logo/cache.py:97-118): global
+ * rows at [0, T) of [B, H, t_cap, D], the last `ring` local rows at slot p %
+ * ring of [B, H, ring, D].  All pointers 16-byte aligned.
+ */
+int logo_cache_prefill(const void* k_local, const void* v_local, const void* k_global, const void* v_global,
+                       void* k_local_cache, void* v_local_cache, void* k_global_cache, void* v_global_cache,
+                       int batch, int h, int64_t n_tokens, int d, int ring, int64_t t_cap, int dtype,
+                       void* stream);
+
+/*
  * Rotary embedding, in place, of up to four [N, H_i, D] bf16 tensors (q, k and
  * the global q, k; a NULL tensor is skipped) with one [N, D] cos / sin pair:
  * x' = x * cos + rotate_half(x) * sin with the eager bf16 rounding of

@@ -55,6 +55,7 @@ SIGNATURES = {
     "logo_decode_fused_workspace_bytes": ([_I, _I, _I, _I], _SZ),
     "logo_decode_attn_fused": ([_P, _P, _P, _P, _I64, _I, _P, _P, _P, _P, _I64, _I, _P, _P, _I, _P, _P, _F, _P, _P, _I,
                                 _I, _I, _I, _F, _I, _P], _I),
+    "logo_cache_prefill": ([_P] * 8 + [_I, _I, _I64, _I, _I, _I64, _I, _P], _I),
     "logo_cache_append": ([_P, _P, _P, _P, _P, _I, _I, _I, _I64, _I, _I, _P], _I),
     "logo_rope_apply": ([_P, _I, _P, _I, _P, _I, _P, _I, _P, _P, _I64, _I, _I, _P], _I),
     "logo_rope": ([_P, _P, _I, _P, _P, _I, _P, _P, _I, _P, _P, _I, _P, _P, _I64, _I, _I, _I, _P], _I),

@@ -172,7 +172,31 @@ class LogoKVCache:
                 self._store_rows(layer, slice(b, b + 1), *(x[b:b + 1].index_select(2, idx)
                                                           for x in (k_local, v_local, k_global, v_global)))
             return
-        self._store_rows(layer, slice(None), k_local, v_local, k_global, v_global)
+        if not self._store_fused(layer, k_local, v_local, k_global, v_global):
+            self._store_rows(layer, slice(None), k_local, v_local, k_global, v_global)
+
+    def _store_fused(self, layer, *rows) -> bool:
+        """``_store_rows`` of a whole batch as one launch, for the layout that
+        the layers pass (``[B, H, T, D]`` views of contiguous 16-bit ``[B, T, H,
+        D]`` tensors, without gradients); False for any other."""
+        caches = (self.local_k[layer], self.local_v[layer], self.global_k[layer], self.global_v[layer])
+        B, H, T, D = rows[0].shape
+        shapes = ((B, H, self.ring, D),) * 2 + ((B, H, self.max_len, D),) * 2
+        dtype = caches[0].dtype
+        if (D not in (64, 128) or T == 0 or B * H > 65535 or dtype not in (torch.bfloat16, torch.float16)
+                or (torch.is_grad_enabled() and any(t.requires_grad for t in (*rows, *caches)))):
+            return False
+        if any(t.shape != rows[0].shape or not t.transpose(1, 2).is_contiguous() for t in rows) or any(
+                tuple(t.shape) != s or not t.is_contiguous() for t, s in zip(caches, shapes)):
+            return False
+        if any(t.device != caches[0].device or not t.is_cuda or t.dtype != dtype or t.data_ptr() % 16
+               for t in (*rows, *caches)):
+            return False
+        lib = _lib.lib()
+        _lib.launch("logo_cache_prefill", lib.logo_cache_prefill, *(_lib.ptr(t) for t in (*rows, *caches)), B, H, T, D,
+                    self.ring, self.max_len, _lib.DTYPE_BF16 if dtype == torch.bfloat16 else _lib.DTYPE_F16,
+                    _lib.stream_of(rows[0]))
+        return True
 
     def _store_rows(self, layer, rows, k_local, v_local, k_global, v_global):
         """Positions [0, T) of batch ``rows``: the global cache, and the last
