@@ -157,7 +157,9 @@ int logo_q_start_blk(const int32_t* pos, const int32_t* cu_q, const int32_t* chu
  * chunk, :348 :413).  Its first
  * bytes are arrival counters that must be zero when a call starts; every call
  * leaves them zero, so one zero-fill serves every later call.  Calls that
- * share a workspace must not overlap.  Too small (or NULL): no split.
+ * share a workspace must not overlap, but for logo_sq_bwd_dq and
+ * logo_sq_bwd_dkv of one call (the same arguments), which use separate parts of
+ * it.  Too small (or NULL): no split.
  */
 int logo_sq_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                 const int64_t* q_idx, const int32_t* pos, const int32_t* meta,
@@ -172,6 +174,9 @@ int logo_sq_fwd(const void* q, const void* k, const void* v, void* o, float* lse
  */
 size_t logo_sq_workspace_bytes(int64_t n_tokens, int nseq, int hq, int d);
 size_t logo_sq_workspace_counter_bytes(void);
+
+/* logo_sq_workspace_bytes for a known number of kv heads (at most that many bytes). */
+size_t logo_sq_kv_workspace_bytes(int64_t n_tokens, int nseq, int hq, int h, int d);
 
 /*
  * The same for head dim 256 in bf16 / fp16 without a window (whose kernels
@@ -212,7 +217,8 @@ int logo_sq_bwd(const void* q, const void* k, const void* v, const void* o,
  * The three backward phases of logo_sq_bwd as separate launches, same
  * arguments: delta and the q_sel / do_sel copies (:124-138, :365-371), dq
  * (:141-228, :424-432), dk/dv (:231-337, :433-445).  Callers time or overlap
- * them one by one; dq and dk/dv read what the delta phase wrote.  Each phase
+ * them one by one; dq and dk/dv read what the delta phase wrote and may run
+ * beside each other, on one workspace too.  Each phase
  * needs only the outputs it writes (dq, or dk and dv); the others may be NULL.
  */
 int logo_sq_bwd_delta(const void* q, const void* k, const void* v, const void* o,

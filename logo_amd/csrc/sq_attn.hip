@@ -198,19 +198,22 @@ using namespace logo;
 
 extern "C" size_t logo_sq_workspace_bytes(int64_t n_tokens, int nseq, int hq, int d) {
   if (n_tokens <= 0 || nseq < 1 || hq < 1 || (d != 64 && d != 128)) return 0;
-  const bool paired = nseq == 1 && n_tokens >= kFwdPairMinTokens;
-  const int cap_f = split_cap_for(hq, paired ? 1 : 2), cap_d = split_cap_for(hq, 2);
-  const size_t fwd = cap_f >= 2 ? (size_t)hq * 2 * cap_f * fwd_part_floats(d, paired ? 8 : 4) : 0;
-  const size_t dq = cap_d >= 2 ? (size_t)hq * 2 * cap_d * dq_part_floats(d) : 0;
-  // dk/dv: at most four pieces a CU for any number of kv heads
-  const size_t dkv = (size_t)4 * device_cus() * dkv_part_floats(d);
-  const size_t part = std::max({fwd, dq, dkv}) * sizeof(float);
-  return part == 0 ? 0 : split_cnt_bytes() + part;
+  size_t dkv = 0;  // for whatever number of kv heads the call has
+  for (int h = 1; h <= hq; ++h)
+    if (hq % h == 0) dkv = std::max(dkv, split_dkv_bytes(n_tokens, nseq, h, d));
+  const size_t part = split_row_bytes(n_tokens, nseq, hq, d) + dkv;
+  return part == 0 ? 0 : 2 * split_cnt_bytes() + part;
+}
+
+extern "C" size_t logo_sq_kv_workspace_bytes(int64_t n_tokens, int nseq, int hq, int h, int d) {
+  if (n_tokens <= 0 || nseq < 1 || h < 1 || hq < h || hq % h != 0 || (d != 64 && d != 128)) return 0;
+  const size_t part = split_row_bytes(n_tokens, nseq, hq, d) + split_dkv_bytes(n_tokens, nseq, h, d);
+  return part == 0 ? 0 : 2 * split_cnt_bytes() + part;
 }
 
 extern "C" size_t logo_sq_wide_workspace_bytes(int hq) { return hq < 1 ? 0 : wide_workspace_bytes(hq); }
 
-extern "C" size_t logo_sq_workspace_counter_bytes(void) { return split_cnt_bytes(); }
+extern "C" size_t logo_sq_workspace_counter_bytes(void) { return 2 * split_cnt_bytes(); }
 
 extern "C" int logo_sq_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                            const int64_t* q_idx, const int32_t* pos, const int32_t* meta,

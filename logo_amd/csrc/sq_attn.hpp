@@ -84,8 +84,12 @@ __host__ __device__ inline int split_pieces(int nt, int cap) {
   return n < kMaxSplit ? n : kMaxSplit;
 }
 
-// Bytes of the arrival counters at the start of the workspace (2 split_cap
-// per head: at most 2 workgroups per CU x 2 rounds x 2), 256-byte aligned.
+// The workspace: [fwd / dq counters][dk/dv counters][fwd / dq partials][dk/dv
+// partials].  dk/dv has counters and partials of its own, so that it may run
+// beside the dq of the same call on one workspace.
+
+// Bytes of one block of arrival counters (2 split_cap per head: at most 2
+// workgroups per CU x 2 rounds x 2), 256-byte aligned.
 inline size_t split_cnt_bytes() { return ((size_t)8 * device_cus() * sizeof(int) + 255) & ~(size_t)255; }
 
 // fp32 partial floats per piece: forward (NW waves: O [DT][16][64] plus m / l
@@ -95,15 +99,66 @@ inline size_t dq_part_floats(int d) { return (size_t)2 * 2 * (d / 32) * 16 * 64;
 // dk/dv: 4 waves x (dK, dV) x [d / 32][16][64]
 inline size_t dkv_part_floats(int d) { return (size_t)4 * 2 * (d / 32) * 16 * 64; }
 
-// Enables the split in `a` when its workspace holds the counters and
+// Whether a call's forward takes two query tiles a workgroup (kFwdPairMinTokens).
+inline bool fwd_paired(int64_t n, int nseq) { return nseq == 1 && n >= kFwdPairMinTokens; }
+
+// Bytes of the fwd / dq partials of a call (d = 64 or 128): 2 split_cap pieces per head.
+inline size_t split_row_bytes(int64_t n, int nseq, int hq, int d) {
+  const bool paired = fwd_paired(n, nseq);
+  const int cap_f = split_cap_for(hq, paired ? 1 : 2), cap_d = split_cap_for(hq, 2);
+  const size_t fwd = cap_f >= 2 ? (size_t)hq * 2 * cap_f * fwd_part_floats(d, paired ? 8 : 4) : 0;
+  const size_t dq = cap_d >= 2 ? (size_t)hq * 2 * cap_d * dq_part_floats(d) : 0;
+  return (fwd > dq ? fwd : dq) * sizeof(float);
+}
+
+// Enables the fwd / dq split in `a` when its workspace holds the counters and
 // 2 split_cap pieces per head of `floats` each; otherwise split_cap = 0.
-inline void split_setup(AttnArgs& a, int heads, int wgs_per_cu, size_t floats) {
-  const int cap = split_cap_for(heads, wgs_per_cu);
-  const size_t need = split_cnt_bytes() + (size_t)heads * 2 * cap * floats * sizeof(float);
+inline void split_setup(AttnArgs& a, int wgs_per_cu, size_t floats) {
+  const int cap = split_cap_for(a.hq, wgs_per_cu);
+  const size_t need = 2 * split_cnt_bytes() + (size_t)a.hq * 2 * cap * floats * sizeof(float);
   if (cap >= 2 && a.ws != nullptr && a.ws_bytes >= need) {
     a.cnt = static_cast<int*>(a.ws);
-    a.part = reinterpret_cast<float*>(static_cast<char*>(a.ws) + split_cnt_bytes());
+    a.part = reinterpret_cast<float*>(static_cast<char*>(a.ws) + 2 * split_cnt_bytes());
     a.split_cap = cap;
+  } else {
+    a.split_cap = 0;
+  }
+}
+
+// Pieces per kv head that dk/dv aims for; 0 where the key blocks of n tokens
+// are too many to be cut.
+inline int dkv_split_cap(int64_t n, int h) {
+  const int cap = split_cap_for(h, 1);
+  return cap >= 2 && 4 * ((n + kBKV - 1) / kBKV) <= 3 * (int64_t)cap ? cap : 0;
+}
+
+// Most workgroups of a kv head over the block counts that n tokens in nseq
+// segments can have: every block once, or all pieces of fewer.
+inline int64_t dkv_ranks(int64_t n, int nseq, int cap) {
+  const int64_t ntmax = (n + (int64_t)(kBKV - 1) * nseq) / kBKV;
+  int64_t ranks = ntmax;
+  for (int nt = 1; nt <= ntmax && 4 * nt <= 3 * cap; ++nt) {
+    const int64_t r = (int64_t)nt * split_pieces(nt, cap);
+    ranks = r > ranks ? r : ranks;
+  }
+  return ranks;
+}
+
+// Bytes of the dk/dv partials of a call with h kv heads (d = 64 or 128).
+inline size_t split_dkv_bytes(int64_t n, int nseq, int h, int d) {
+  const int cap = dkv_split_cap(n, h);
+  return cap == 0 ? 0 : (size_t)h * dkv_ranks(n, nseq, cap) * dkv_part_floats(d) * sizeof(float);
+}
+
+// Enables the dk/dv split in `a` (head dim d) when its workspace reaches behind
+// the fwd / dq partials of the same call; otherwise split_cap = 0.
+inline void split_setup_dkv(AttnArgs& a, int d) {
+  const size_t at = 2 * split_cnt_bytes() + split_row_bytes(a.n, a.nseq, a.hq, d);
+  const size_t bytes = split_dkv_bytes(a.n, a.nseq, a.h, d);
+  if (bytes != 0 && a.ws != nullptr && a.ws_bytes >= at + bytes) {
+    a.cnt = reinterpret_cast<int*>(static_cast<char*>(a.ws) + split_cnt_bytes());
+    a.part = reinterpret_cast<float*>(static_cast<char*>(a.ws) + at);
+    a.split_cap = dkv_split_cap(a.n, a.h);
   } else {
     a.split_cap = 0;
   }

@@ -4,8 +4,6 @@
 // through LDS, dK / dV of the whole group stored once in bf16.
 #include "sq_attn.hpp"
 
-#include <algorithm>
-
 namespace logo {
 
 // ---------------------------------------------------------------------------
@@ -471,7 +469,8 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
     // partial dK and dV of this piece as [wave][dK, dV][dt][item][lane]; the
     // last piece of the key block to arrive adds all of them in piece order
     constexpr int PW = 2 * DT * 16 * 64;  // floats per wave
-    float* const part0 = a.part + (int64_t)(h * 2 * a.split_cap + tile * nper) * 4 * PW + wave * PW + l;
+    const int ranks = gridDim.x / a.h;  // pieces per head in the workspace (dkv_ranks)
+    float* const part0 = a.part + ((int64_t)h * ranks + tile * nper) * 4 * PW + wave * PW + l;
     {
       float* pp = part0 + (int64_t)piece * 4 * PW;
 #pragma unroll
@@ -546,10 +545,9 @@ constexpr size_t dkv_smem() { return (size_t)kDkvStages * dkv_stage_bytes<D>(); 
 template <typename EL, int D, bool SPARSE, bool WINDOW>
 static int launch_dkv(const AttnArgs& a_in, hipStream_t st) {
   AttnArgs a = a_in;
-  const int64_t ntmax = (a.n + kBKV - 1) / kBKV + a.nseq;
   if (WINDOW) a.split_cap = 0;
-  else split_setup(a, a.h, 1, dkv_part_floats(D));
-  const int64_t nblk = std::max<int64_t>(ntmax, 2 * a.split_cap) * a.h;
+  else split_setup_dkv(a, D);
+  const int64_t nblk = dkv_ranks(a.n, a.nseq, a.split_cap) * a.h;
   LOGO_REQUIRE(nblk < ((int64_t)1 << 31), "grid too large");
   auto kern = sq_dkv_kernel<EL, D, SPARSE, WINDOW>;
   LOGO_HIP_CHECK(allow_smem(kern, dkv_smem<D>()));

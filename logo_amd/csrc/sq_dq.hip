@@ -355,7 +355,7 @@ static int launch_dq(const AttnArgs& a_in, hipStream_t st) {
   AttnArgs a = a_in;
   const int64_t ntmax = (a.n + kBQ - 1) / kBQ + a.nseq;
   if (WINDOW) a.split_cap = 0;
-  else split_setup(a, a.hq, 2, dq_part_floats(D));
+  else split_setup(a, 2, dq_part_floats(D));
   const int64_t nblk = std::max<int64_t>(ntmax, 2 * a.split_cap) * a.hq;
   LOGO_REQUIRE(nblk < ((int64_t)1 << 31), "grid too large");
   auto kern = sq_dq64_kernel<EL, D, SPARSE, WINDOW>;

@@ -375,11 +375,11 @@ constexpr size_t fwd_smem() { return (size_t)4 * TileGeom<D, kSwz>::ELEMS * size
 template <typename EL, int D, bool SPARSE, bool WINDOW>
 static int launch_fwd(const AttnArgs& a_in, hipStream_t st) {
   AttnArgs a = a_in;
-  const bool paired = a.nseq == 1 && a.n >= kFwdPairMinTokens;
+  const bool paired = fwd_paired(a.n, a.nseq);
   const int64_t rows = paired ? 2 * kBQ : kBQ;
   const int64_t ntmax = (a.n + rows - 1) / rows + a.nseq;
   if (WINDOW) a.split_cap = 0;
-  else split_setup(a, a.hq, paired ? 1 : 2, fwd_part_floats(D, paired ? 8 : 4));
+  else split_setup(a, paired ? 1 : 2, fwd_part_floats(D, paired ? 8 : 4));
   const int64_t nblk = std::max<int64_t>(ntmax, 2 * a.split_cap) * a.hq;
   LOGO_REQUIRE(nblk < ((int64_t)1 << 31), "grid too large");
   if (paired) {

@@ -880,7 +880,7 @@ constexpr size_t kRowSmem = (size_t)4 * GT::ELEMS * sizeof(bf16);
 template <typename EL, bool SPARSE>
 int launch_rows(const AttnArgs& a_in, hipStream_t st, bool bwd) {
   AttnArgs a = a_in;
-  split_setup(a, a.hq, 1, bwd ? dq_part_floats(D) : fwd_part_floats(D, 4));
+  split_setup(a, 1, bwd ? dq_part_floats(D) : fwd_part_floats(D, 4));
   a.round_rows /= 2;  // one 128-row workgroup per CU in a round
   const int64_t nblk = std::max<int64_t>((a.n + kBQ - 1) / kBQ + a.nseq, 2 * a.split_cap) * a.hq;
   LOGO_REQUIRE(nblk < ((int64_t)1 << 31), "grid too large");
@@ -918,7 +918,7 @@ bool wide_applies(const AttnArgs& a, int d, int dtype) {
 size_t wide_workspace_bytes(int hq) {
   const int cap = split_cap_for(hq, 1);
   if (cap < 2) return 0;
-  return split_cnt_bytes() +
+  return 2 * split_cnt_bytes() +
          (size_t)hq * 2 * cap * std::max(fwd_part_floats(wide::D, 4), dq_part_floats(wide::D)) * sizeof(float);
 }
 

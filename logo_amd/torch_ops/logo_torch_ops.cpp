@@ -98,13 +98,17 @@ int check_attn(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
   return dt == at::kHalf ? LOGO_DTYPE_F16 : dt == at::kFloat ? LOGO_DTYPE_F32 : LOGO_DTYPE_BF16;
 }
 
-// Whether the call runs on the generic kernels (no compacted copies, no split).
+// Whether the call's backward reads q and dO in place (no compacted copies):
+// head dim 256 and fp32.
 bool generic_path(const at::Tensor& q, int dtype) { return logo_sq_generic((int)q.size(2), dtype) != 0; }
 
-// Split workspace of the fwd / dq kernels for this shape (empty: no split).
-// Its size depends only on the device's CU count, HQ and D (the pieces a
-// split aims for fill the device twice, whatever N is): at most 136 MB at
-// D = 128 on MI355X.
+// Split workspace of the fwd, dq and dk/dv kernels for this shape (empty: no
+// split).  Calls on one buffer must not overlap, except dk/dv with the dq of
+// its own call, whose counters and partials are apart.  The part of fwd and dq
+// depends only on the device's CU count, HQ and D (the pieces a split aims for
+// fill the device twice, whatever N is): at most 136 MB at D = 128 on MI355X,
+// also at D = 256; that of dk/dv, at most 118 MB at D = 128, is there only
+// where its key blocks are few enough to be cut.
 //  * Outside graph capture: one buffer per (device, stream), kept across
 //    calls and grown on demand.  The kernels leave its counter prefix zero,
 //    so only a new buffer needs the zero fill, and calls on one stream run in
@@ -121,12 +125,13 @@ bool generic_path(const at::Tensor& q, int dtype) { return logo_sq_generic((int)
 // and tests that compare kernel variants bit for bit).
 constexpr size_t kMaxCachedStreams = 16;
 
-at::Tensor split_workspace(const at::Tensor& q, const at::Tensor& cu, int dtype) {
+at::Tensor split_workspace(const at::Tensor& q, const at::Tensor& k, const at::Tensor& cu, int dtype) {
   const char* env = std::getenv("LOGO_SQ_SPLIT");
   size_t bytes = 0;
   if (env == nullptr || env[0] != '0') {
     if (!generic_path(q, dtype))
-      bytes = logo_sq_workspace_bytes(q.size(0), (int)cu.numel() - 1, (int)q.size(1), (int)q.size(2));
+      bytes = logo_sq_kv_workspace_bytes(q.size(0), (int)cu.numel() - 1, (int)q.size(1), (int)k.size(1),
+                                         (int)q.size(2));
     else if (dtype != LOGO_DTYPE_F32)
       bytes = logo_sq_wide_workspace_bytes((int)q.size(1));
   }
@@ -167,7 +172,7 @@ std::tuple<at::Tensor, at::Tensor> sq_fwd(const at::Tensor& q, const at::Tensor&
   // tokens and for lse rows past each lane's rows, by the kernel).
   auto o = at::empty_like(q);
   auto lse = at::empty({hq, n}, q.options().dtype(at::kFloat));
-  auto ws = window < 0 ? split_workspace(q, cu, dtype) : at::empty({0}, q.options().dtype(at::kByte));
+  auto ws = window < 0 ? split_workspace(q, k, cu, dtype) : at::empty({0}, q.options().dtype(at::kByte));
   ok(logo_sq_fwd(cptr(q), cptr(k), cptr(v), mptr(o), lse.data_ptr<float>(), opt_ptr<int64_t>(q_idx),
                  opt_ptr<int32_t>(pos), meta.data_ptr<int32_t>(), cu.data_ptr<int32_t>(), n, (int)cu.numel() - 1,
                  (int)hq, (int)h, (int)d, (int)v.size(2), (int)lanes, (float)scale, (int)window, dtype,
@@ -204,8 +209,8 @@ struct Bwd {
     F fn = phase == 0 ? &logo_sq_bwd_delta : phase == 1 ? &logo_sq_bwd_dq : phase == 2 ? &logo_sq_bwd_dkv
                                                                                   : &logo_sq_bwd_dqkv;
     auto p = [](at::Tensor* t) -> void* { return t && t->numel() ? t->data_ptr() : nullptr; };
-    at::Tensor ws = phase >= 1 && window < 0 ? split_workspace(q, cu, dtype)
-                                                            : at::empty({0}, q.options().dtype(at::kByte));
+    at::Tensor ws = phase >= 1 && window < 0 ? split_workspace(q, k, cu, dtype)
+                                             : at::empty({0}, q.options().dtype(at::kByte));
     return fn(cptr(q), cptr(k), cptr(v), cptr(o), cptr(dout), lse.data_ptr<float>(),
               static_cast<float*>(p(delta)), p(q_sel), p(do_sel), p(dq), p(dk), p(dv), opt_ptr<int64_t>(q_idx),
               opt_ptr<int32_t>(pos), meta.data_ptr<int32_t>(), cu.data_ptr<int32_t>(), q.size(0),
