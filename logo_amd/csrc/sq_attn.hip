@@ -200,14 +200,14 @@ extern "C" size_t logo_sq_workspace_bytes(int64_t n_tokens, int nseq, int hq, in
   if (n_tokens <= 0 || nseq < 1 || hq < 1 || (d != 64 && d != 128)) return 0;
   size_t dkv = 0;  // for whatever number of kv heads the call has
   for (int h = 1; h <= hq; ++h)
-    if (hq % h == 0) dkv = std::max(dkv, split_dkv_bytes(n_tokens, nseq, h, d));
+    if (hq % h == 0) dkv = std::max(dkv, split_dkv_bytes(n_tokens, nseq, hq, h, d));
   const size_t part = split_row_bytes(n_tokens, nseq, hq, d) + dkv;
   return part == 0 ? 0 : 2 * split_cnt_bytes() + part;
 }
 
 extern "C" size_t logo_sq_kv_workspace_bytes(int64_t n_tokens, int nseq, int hq, int h, int d) {
   if (n_tokens <= 0 || nseq < 1 || h < 1 || hq < h || hq % h != 0 || (d != 64 && d != 128)) return 0;
-  const size_t part = split_row_bytes(n_tokens, nseq, hq, d) + split_dkv_bytes(n_tokens, nseq, h, d);
+  const size_t part = split_row_bytes(n_tokens, nseq, hq, d) + split_dkv_bytes(n_tokens, nseq, hq, h, d);
   return part == 0 ? 0 : 2 * split_cnt_bytes() + part;
 }
 

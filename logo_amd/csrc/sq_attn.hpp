@@ -125,11 +125,32 @@ inline void split_setup(AttnArgs& a, int wgs_per_cu, size_t floats) {
   }
 }
 
-// Pieces per kv head that dk/dv aims for; 0 where the key blocks of n tokens
-// are too many to be cut.
-inline int dkv_split_cap(int64_t n, int h) {
+// Query rows that dk/dv stages per step.
+constexpr int kDkvRows = 128;
+
+// Fewest steps of a piece of a dk/dv key block, where a kv head has nt of them
+// and cap is two workgroups a CU (one CU holds one).  A piece starts like a
+// block (8 to 10 us with the loads of K and V) and writes 128 KB of partials at
+// D = 128, so pieces pay while CUs are idle; beyond one block a CU they have to
+// be long enough to make up for a second round.  A block with fewer than two
+// times these steps is left whole.  dk/dv alone, cut against whole, D = 64 and
+// 128, 2 to 16 kv heads, 500 to 24000 tokens, one and six segments:
+//   blocks below half the CUs (3): 6 to 11 steps in the heaviest block 0.78x,
+//     12 to 25 0.52x, 64 and more 0.35x
+//   up to one a CU (16): 26 to 39 steps 0.80x, 64 and more 0.75x; cut into pieces
+//     of 5 steps, 12 to 17 steps took up to 1.24x
+//   up to 9/8 of them (24): 64 to 99 steps 0.91x, from 100 on 0.73x
+//   up to 3/2 (96): from 176 steps on 0.90x; pieces of 24 steps up to 1.23x
+constexpr int dkv_min_steps(int nt, int cap) {
+  return 4 * nt < cap ? 3 : 2 * nt <= cap ? 16 : 16 * nt <= 9 * cap ? 24 : 96;
+}
+
+// Pieces per kv head that dk/dv aims for; 0 where no block of n tokens can be
+// cut: too many blocks, or too few steps with every row selected.
+inline int dkv_split_cap(int64_t n, int hq, int h) {
   const int cap = split_cap_for(h, 1);
-  return cap >= 2 && 4 * ((n + kBKV - 1) / kBKV) <= 3 * (int64_t)cap ? cap : 0;
+  const int64_t nt = (n + kBKV - 1) / kBKV, steps = hq / h * ((n + kDkvRows - 1) / kDkvRows);
+  return cap >= 2 && 4 * nt <= 3 * (int64_t)cap && steps >= 2 * dkv_min_steps((int)nt, cap) ? cap : 0;
 }
 
 // Most workgroups of a kv head over the block counts that n tokens in nseq
@@ -144,9 +165,9 @@ inline int64_t dkv_ranks(int64_t n, int nseq, int cap) {
   return ranks;
 }
 
-// Bytes of the dk/dv partials of a call with h kv heads (d = 64 or 128).
-inline size_t split_dkv_bytes(int64_t n, int nseq, int h, int d) {
-  const int cap = dkv_split_cap(n, h);
+// Bytes of the dk/dv partials of a call (d = 64 or 128).
+inline size_t split_dkv_bytes(int64_t n, int nseq, int hq, int h, int d) {
+  const int cap = dkv_split_cap(n, hq, h);
   return cap == 0 ? 0 : (size_t)h * dkv_ranks(n, nseq, cap) * dkv_part_floats(d) * sizeof(float);
 }
 
@@ -154,11 +175,11 @@ inline size_t split_dkv_bytes(int64_t n, int nseq, int h, int d) {
 // the fwd / dq partials of the same call; otherwise split_cap = 0.
 inline void split_setup_dkv(AttnArgs& a, int d) {
   const size_t at = 2 * split_cnt_bytes() + split_row_bytes(a.n, a.nseq, a.hq, d);
-  const size_t bytes = split_dkv_bytes(a.n, a.nseq, a.h, d);
+  const size_t bytes = split_dkv_bytes(a.n, a.nseq, a.hq, a.h, d);
   if (bytes != 0 && a.ws != nullptr && a.ws_bytes >= at + bytes) {
     a.cnt = reinterpret_cast<int*>(static_cast<char*>(a.ws) + split_cnt_bytes());
     a.part = reinterpret_cast<float*>(static_cast<char*>(a.ws) + at);
-    a.split_cap = dkv_split_cap(a.n, a.h);
+    a.split_cap = dkv_split_cap(a.n, a.hq, a.h);
   } else {
     a.split_cap = 0;
   }

@@ -9,16 +9,12 @@ namespace logo {
 // ---------------------------------------------------------------------------
 // Backward dk / dv
 // ---------------------------------------------------------------------------
-// Query rows staged per LDS buffer: two 64-row sub-tiles per step, half the
+// kDkvRows query rows a step and LDS buffer: two 64-row sub-tiles, half the
 // barriers, copy issues and step bookkeeping per row of 64-row steps.  Two
 // stages take 131 KB (one workgroup per CU, as its registers already allow);
 // the second stage's LDS addresses lie past the 64 KB reach of the
 // instruction offset, so the compiler keeps them in spare AGPRs.
-constexpr int kDkvRows = 128;
 constexpr int kDkvStages = 2;
-// Fewest steps a piece of a split key block takes: its partials cost about one
-// (128 KB at D = 128, written and read back).
-constexpr int kDkvMinSteps = 3;
 template <int D>
 constexpr int dkv_stage_bytes() { return 2 * kDkvRows * D * 2 + 3 * kDkvRows * 4; }
 
@@ -45,8 +41,14 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
   const int ntk = meta0[2];
   const int nper = WINDOW ? 1 : split_pieces(ntk, a.split_cap);
   if (rank >= ntk * nper) return;
-  const int tile = rank / nper;  // early key blocks (most queries) first
-  const int piece = rank - tile * nper;
+  // early key blocks (most queries) first; the first pieces of all blocks ahead
+  // of the others, so that workgroups without a piece, where the blocks have too
+  // few steps, come when the others run
+  const int piece = rank / ntk;
+  const int tile = rank - piece * ntk;
+  const int min_steps = dkv_min_steps(ntk, a.split_cap);
+  const int32_t* meta_h = meta0 + (int64_t)(a.lanes > 1 ? h * a.g : 0) * a.meta_stride;  // the group's first head
+  if (piece > 0 && (meta_h[0] + RS - 1) / RS * a.g < 2 * min_steps) return;
   const int32_t* cu_tk = meta0 + kMetaHdr + 2 * (a.nseq + 1);
   const int s = seg_of(cu_tk, a.nseq, tile);
   const int k0 = (tile - cu_tk[s]) * kBKV;
@@ -55,30 +57,22 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
   const int k_last = min(k0 + kBKV, seqlen) - 1;
 
   // Row-range split of a key block (no window), where the kv heads have few
-  // key blocks (at most 3/4 of two workgroups a CU): the steps of all query
-  // heads of the group, one after the other, are cut into nsplit runs of at
-  // least kDkvMinSteps; this piece takes steps [st_lo, st_hi).  One workgroup a
-  // block left the GPU to its heaviest blocks (16 query, 4 kv heads of dim 64,
-  // 6001 tokens: 188 blocks of 1 to 48 steps on 256 CUs; forward + backward 215
-  // -> 183 us; 8 query, 2 kv heads, 4000 tokens, rows per head: 295 -> 186).
-  int nsplit = 1, st_lo = 0, st_hi = 0x7fffffff;
+  // key blocks (at most 3/4 of two workgroups a CU) and one workgroup a block
+  // would leave the GPU to its heaviest blocks: the steps of all query heads of
+  // the group, one after the other, are cut into nsplit equal runs of at least
+  // dkv_min_steps, counted at the group's first head; this piece takes run
+  // `piece`.  What a block that stays whole pays for the rule: under 0.4 us.
+  int nsplit = 1;
   if (nper > 1) {
-    int total = 0;
-    for (int gg = 0; gg < a.g; ++gg) {
-      const int lane_sel = a.lanes > 1 ? h * a.g + gg : 0;
-      const int32_t* cu_q = a.meta + (int64_t)lane_sel * a.meta_stride + kMetaHdr;
-      const int lo = cu_q[s], hi = cu_q[s + 1];
-      const int r0 = SPARSE ? wave_lower_bound(row_view<SPARSE>(a, lane_sel, bos).ps, lo, hi, k0) : min(lo + k0, hi);
-      total += (hi - r0 + RS - 1) / RS;
-      if (a.lanes == 1) {  // every head has these rows
-        total *= a.g;
-        break;
-      }
+    const int lo = meta_h[kMetaHdr + s], hi = meta_h[kMetaHdr + s + 1];
+    int total = (hi - lo + RS - 1) / RS * a.g;
+    if (total >= 2 * min_steps) {
+      const int r0 = SPARSE ? wave_lower_bound(row_view<SPARSE>(a, a.lanes > 1 ? h * a.g : 0, bos).ps, lo, hi, k0)
+                            : min(lo + k0, hi);
+      total = (hi - r0 + RS - 1) / RS * a.g;
     }
-    nsplit = max(1, min(nper, total / kDkvMinSteps));
+    nsplit = max(1, min(nper, total / min_steps));
     if (piece >= nsplit) return;
-    st_lo = total * piece / nsplit;
-    st_hi = total * (piece + 1) / nsplit;
   }
 
   const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, i = l & 31, g = l >> 5;
@@ -123,6 +117,10 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
   float lse_n = 0.f, delta_n = 0.f;
   int pos_n = -1;
   for (int gg = 0; gg < a.g; ++gg) {
+    // this piece's share of the head: steps [steps sh_lo / nsplit, steps sh_hi / nsplit)
+    const int sh_lo = min(max(piece * a.g - gg * nsplit, 0), nsplit);
+    const int sh_hi = min(max((piece + 1) * a.g - gg * nsplit, 0), nsplit);
+    if (nsplit > 1 && sh_lo == sh_hi) continue;
     const int hq = h * a.g + gg;
     const int lane_sel = a.lanes > 1 ? hq : 0;
     const int32_t* cu_q = a.meta + (int64_t)lane_sel * a.meta_stride + kMetaHdr;
@@ -136,13 +134,11 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
     };
     int rq0 = lb_pos(q_lo, q_hi, k0);
     int rq_end = WINDOW ? lb_pos(rq0, q_hi, k_last + W + 1) : q_hi;
-    if (nsplit > 1) {  // this piece's share of the head's steps
+    if (nsplit > 1) {
       const int steps = (rq_end - rq0 + RS - 1) / RS;
-      const int lo = min(max(st_lo, 0), steps), hi = min(max(st_hi, 0), steps);
+      const int lo = steps * sh_lo / nsplit, hi = steps * sh_hi / nsplit;
       rq_end = min(rq_end, rq0 + RS * hi);
       rq0 = min(rq_end, rq0 + RS * lo);
-      st_lo -= steps;
-      st_hi -= steps;
     }
     // This wave's keys kw0 .. kw_last: rows before lb0 see none of them,
     // rows from lb1 on see all of them (causally), rows from lb2 on are past
