@@ -79,6 +79,17 @@ class LoGoConfig:
         return self.hidden_size // self.num_attention_heads
 
 
+#: The ``forward`` of each module class whose arithmetic a decode step does itself.
+_OWN_FORWARD = {nn.Linear: nn.Linear.forward}
+
+
+def own_forward(cls):
+    """Class decorator: ``_plain`` knows the class by the ``forward`` it has now."""
+    _OWN_FORWARD[cls] = cls.forward
+    return cls
+
+
+@own_forward
 class RMSNorm(nn.Module):
     """RMSNorm with the reference's rounding order (logo/modules/layernorm.py:9-22)."""
 
@@ -104,24 +115,29 @@ def _fused_ok(*tensors) -> bool:
     return all(t.is_cuda and t.dtype == torch.bfloat16 for t in tensors)
 
 
-def _unhooked(*modules) -> bool:
-    """Whether calling the modules' own arithmetic directly is what calling
-    them would do: no forward hook of theirs or of every module is skipped."""
-    return not torch.nn.modules.module._has_any_global_hook() and not any(
-        m._forward_hooks or m._forward_pre_hooks for m in modules)
+def _plain(*modules) -> bool:
+    """Whether doing the modules' own arithmetic directly is what calling them
+    would do: no forward hook of theirs or of every module, no subclass, and no
+    ``forward`` put in the place of the class's own, on the instance (as tools
+    that wrap a model do) or on the class."""
+    return not torch.nn.modules.module._has_any_global_hook() and all(
+        type(m).forward is _OWN_FORWARD.get(type(m)) and "forward" not in m.__dict__
+        and not m._forward_hooks and not m._forward_pre_hooks for m in modules)
 
 
 def _dec_weight_ok(rows: int, w) -> bool:
     """Whether ``dec_linear`` serves ``rows`` input rows of a bias-free linear
-    layer with weight ``w`` (inference, outside autocast)."""
-    return (dec_linear_ok(rows, w) and _fused_ok(w) and not torch.is_autocast_enabled("cuda"))
+    layer with weight ``w``, a plain tensor (inference, outside autocast)."""
+    return (type(w) in (torch.Tensor, nn.Parameter) and dec_linear_ok(rows, w) and _fused_ok(w)
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def linear_rows(lin: nn.Linear, x):
     """``lin(x)``, on ``dec_linear`` for the few rows of a decode step."""
-    w = lin.weight
-    if type(lin) is nn.Linear and lin.bias is None and x.numel() <= 16 * x.shape[-1] and _fused_ok(x, w) \
-            and x.shape[-1] == w.shape[1] and _dec_weight_ok(x.numel() // x.shape[-1], w) and _unhooked(lin):
+    if not (_plain(lin) and type(lin) is nn.Linear and lin.bias is None and type(x) is torch.Tensor):
+        return lin(x)
+    w, k = lin.weight, x.shape[-1]
+    if 0 < x.numel() <= 16 * k and k == w.shape[1] and _fused_ok(x, w) and _dec_weight_ok(x.numel() // k, w):
         return dec_linear(x, w)
     return lin(x)
 
@@ -270,6 +286,7 @@ def _per_head_linear(x, w):
     return y.transpose(0, 1).reshape(*lead, H, w.shape[-1]).contiguous()
 
 
+@own_forward
 class LoGoAttention(nn.Module):
     """Token-level dynamic local-global attention (logo/layers/logo.py:34-262)."""
 

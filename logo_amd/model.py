@@ -21,14 +21,15 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .layers import (Attention, LoGoAttention, LoGoConfig, RMSNorm, _dec_weight_ok, _fused_ok, _unhooked, linear_rows,
-                     padding_mask, position_ids_for, rope_cos_sin)
+from .layers import (Attention, LoGoAttention, LoGoConfig, RMSNorm, _dec_weight_ok, _fused_ok, _plain, linear_rows,
+                     own_forward, padding_mask, position_ids_for, rope_cos_sin)
 from .ops.decode import LogoKVCache
 from .ops.glue import add_rms_norm, dec_linear, silu_mul
 
 __all__ = ["LoGoMLP", "LoGoDecoderLayer", "LoGoModel", "LoGoForCausalLM"]
 
 
+@own_forward
 class LoGoMLP(nn.Module):
     """SwiGLU feed-forward (logo/modules/mlp.py:10-27, ``hidden_act = silu``)."""
 
@@ -55,6 +56,7 @@ class LoGoMLP(nn.Module):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
+@own_forward
 class LoGoDecoderLayer(nn.Module):
     """Pre-norm attention + MLP block (logo/modeling_logo.py:42-106); the
     attention is LoGo's or plain per ``config.attn_type_list``."""
@@ -82,7 +84,7 @@ class LoGoDecoderLayer(nn.Module):
         lins = (a.q_proj, a.k_proj, a.v_proj, a.gate_proj, a.o_proj, m.gate_proj, m.up_proj, m.down_proj)
         if any(type(x) is not nn.Linear or x.bias is not None for x in lins) or m.up_proj.weight.shape[0] % 8:
             return False
-        return (_unhooked(self, a, m, *norms, *lins) and a._fused_decode_ok(h, cache)
+        return (_plain(self, a, m, *norms, *lins) and a._fused_decode_ok(h, cache)
                 and _fused_ok(*(n.weight for n in norms), *(x.weight for x in lins))
                 and all(_dec_weight_ok(h.shape[0], x.weight) for x in (a.q_proj, a.o_proj, m.up_proj, m.down_proj)))
 

@@ -77,3 +77,66 @@ def test_hooks_and_other_modules_keep_their_calls(gpu):
         logits.append(model.decode_step(tok, cache).double())
     assert len(calls) == 3
     assert float((logits[0] - logits[1]).norm() / logits[1].norm()) <= 2e-2
+
+
+def _model(gpu, **kw):
+    from logo_amd.layers import LoGoConfig
+    from logo_amd.model import LoGoForCausalLM
+
+    cfg = LoGoConfig(**{"vocab_size": 256, "hidden_size": 256, "intermediate_size": 512, "num_hidden_layers": 2,
+                        "num_attention_heads": 4, "gate_thres_init": -1.0, **kw})
+    model = LoGoForCausalLM(cfg)
+    model.init_weights(torch.Generator().manual_seed(0))
+    return model.to(device=gpu, dtype=torch.bfloat16).eval()
+
+
+def _step(model, gpu, rows=3):
+    ids = torch.randint(0, 256, (rows, 40), generator=torch.Generator().manual_seed(1)).to(gpu)
+    cache = model.new_cache(rows, 60, device=gpu)
+    model.prefill(ids, cache)
+    return model.decode_step(ids[:, 0].clone(), cache)
+
+
+@pytest.mark.parametrize("where", ["mlp", "self_attn", "o_proj", "down_proj", "lm_head"])
+def test_a_forward_set_on_an_instance_is_called(gpu, where):
+    """A decode step runs the replacement that a wrapping tool puts on a module,
+    as the prefill before it does: here one that doubles the module's output."""
+    model = _model(gpu)
+    layer = model.model.layers[1]
+    mod = {"mlp": layer.mlp, "self_attn": layer.self_attn, "o_proj": layer.self_attn.o_proj,
+           "down_proj": layer.mlp.down_proj, "lm_head": model.lm_head}[where]
+    want = _step(model, gpu)
+    calls, own = [], mod.forward
+
+    def wrapped(*args, **kw):
+        calls.append(args[0].shape[1] if args[0].dim() == 3 else 1)
+        out = own(*args, **kw)
+        return (2 * out[0], *out[1:]) if isinstance(out, tuple) else 2 * out
+
+    mod.forward = wrapped
+    got = _step(model, gpu)
+    assert 1 in calls, f"{where}: the decode step skipped the replacement"
+    if where == "lm_head":
+        assert torch.equal(got, 2 * want)
+    else:
+        assert float((got.double() - want.double()).norm() / want.double().norm()) > 2e-2
+
+
+class _Scaled(torch.Tensor):
+    """A weight whose layer computes something else: linear() doubles its result."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        out = super().__torch_function__(func, types, args, kwargs or {})
+        return 2 * out.as_subclass(torch.Tensor) if func is torch.nn.functional.linear else out
+
+
+def test_weights_of_a_tensor_subclass_keep_their_arithmetic(gpu):
+    from logo_amd.layers import linear_rows
+
+    lin = torch.nn.Linear(256, 64, bias=False).to(device=gpu, dtype=torch.bfloat16)
+    x = torch.randn(2, 256, device=gpu).bfloat16()
+    with torch.no_grad():
+        want = 2 * torch.nn.functional.linear(x, lin.weight)
+        lin.weight = torch.nn.Parameter(lin.weight.detach().as_subclass(_Scaled), requires_grad=False)
+        assert torch.equal(linear_rows(lin, x), want)
