@@ -30,7 +30,7 @@ import torch.nn.functional as F
 from .ops.decode import LogoKVCache, decode_attn, decode_attn_fused, decode_qkv
 from .ops.epilogue import logo_epilogue
 from .ops.glue import (attn_inputs, dec_linear, dec_linear_ok, global_maps_, global_maps_ok, head_linear, head_proj,
-                       rms_norm, rope, rope_apply_)
+                       rms_norm, rope, rope_apply_, silu_mul)
 from .ops.sq_attn import dense_causal_attn, sq_full_attn, swa_attn
 
 __all__ = ["LoGoConfig", "LoGoAttention", "Attention", "RMSNorm", "rope_cos_sin", "apply_rope", "position_ids_for"]
@@ -125,20 +125,30 @@ def _plain(*modules) -> bool:
         and not m._forward_hooks and not m._forward_pre_hooks for m in modules)
 
 
-def _dec_weight_ok(rows: int, w) -> bool:
-    """Whether ``dec_linear`` serves ``rows`` input rows of a bias-free linear
-    layer with weight ``w``, a plain tensor (inference, outside autocast)."""
-    return (type(w) in (torch.Tensor, nn.Parameter) and dec_linear_ok(rows, w) and _fused_ok(w)
-            and not torch.is_autocast_enabled("cuda"))
+def rows_product(x, w, norm=None, resid=None, glu=False):
+    """``x w^T`` for the rows of a decode step (bf16, no gradients), with the
+    RMSNorm ``norm`` before it and the add of ``resid`` or the SwiGLU of a
+    stacked gate / up weight behind it: one launch where ``dec_linear`` serves
+    the weight (a plain tensor, outside autocast), else the library's product and
+    a launch each."""
+    k = w.shape[1]
+    rows = x.numel() // k
+    if (type(x) is torch.Tensor and type(w) in (torch.Tensor, nn.Parameter) and x.shape[-1] == k
+            and dec_linear_ok(rows, w) and not torch.is_autocast_enabled("cuda")):
+        if norm is None:
+            return dec_linear(x, w, resid=resid, glu=glu)
+        return dec_linear(x, w, norm_w=norm.weight, eps=norm.variance_epsilon, resid=resid, glu=glu)
+    y = F.linear(x if norm is None else rms_norm(x, norm.weight, norm.variance_epsilon), w)
+    if glu:
+        return silu_mul(y)
+    return y if resid is None else resid + y
 
 
 def linear_rows(lin: nn.Linear, x):
     """``lin(x)``, on ``dec_linear`` for the few rows of a decode step."""
-    if not (_plain(lin) and type(lin) is nn.Linear and lin.bias is None and type(x) is torch.Tensor):
-        return lin(x)
-    w, k = lin.weight, x.shape[-1]
-    if 0 < x.numel() <= 16 * k and k == w.shape[1] and _fused_ok(x, w) and _dec_weight_ok(x.numel() // k, w):
-        return dec_linear(x, w)
+    if 0 < x.numel() <= 16 * x.shape[-1] and _plain(lin) and type(lin) is nn.Linear and lin.bias is None \
+            and _fused_ok(x, lin.weight):
+        return rows_product(x, lin.weight)
     return lin(x)
 
 
@@ -411,8 +421,7 @@ class LoGoAttention(nn.Module):
         """Decode step with the stacked q / k / v / gate GEMM and one launch for
         the global projections, RoPE and cache appends (same arithmetic as the
         step-by-step path: the same roundings, in the same order)."""
-        w = self._decode_weight()
-        qkv = dec_linear(hidden_states, w) if _dec_weight_ok(hidden_states.shape[0], w) else F.linear(hidden_states, w)
+        qkv = rows_product(hidden_states, self._decode_weight())
         return self._decode_rows(qkv, cache, position_embeddings, position_ids)
 
     def _decode_rows(self, qkv, cache: LogoKVCache, position_embeddings, position_ids):

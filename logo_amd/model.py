@@ -21,10 +21,10 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .layers import (Attention, LoGoAttention, LoGoConfig, RMSNorm, _dec_weight_ok, _fused_ok, _plain, linear_rows,
-                     own_forward, padding_mask, position_ids_for, rope_cos_sin)
+from .layers import (Attention, LoGoAttention, LoGoConfig, RMSNorm, _fused_ok, _plain, linear_rows, own_forward,
+                     padding_mask, position_ids_for, rope_cos_sin, rows_product)
 from .ops.decode import LogoKVCache
-from .ops.glue import add_rms_norm, dec_linear, silu_mul
+from .ops.glue import DEC_LINEAR_MAX_ROWS, add_rms_norm, silu_mul
 
 __all__ = ["LoGoMLP", "LoGoDecoderLayer", "LoGoModel", "LoGoForCausalLM"]
 
@@ -76,6 +76,8 @@ class LoGoDecoderLayer(nn.Module):
     def _decode_ok(self, h, cache) -> bool:
         """Whether a decode step of this layer runs as ``_decode_step``: plain
         modules without hooks, few rows, bf16 inference."""
+        if h.shape[0] > DEC_LINEAR_MAX_ROWS or torch.is_autocast_enabled("cuda"):
+            return False
         a, m = self.self_attn, self.mlp
         norms = (self.input_layernorm, self.post_attention_layernorm)
         if type(self) is not LoGoDecoderLayer or type(a) is not LoGoAttention or type(m) is not LoGoMLP \
@@ -85,19 +87,17 @@ class LoGoDecoderLayer(nn.Module):
         if any(type(x) is not nn.Linear or x.bias is not None for x in lins) or m.up_proj.weight.shape[0] % 8:
             return False
         return (_plain(self, a, m, *norms, *lins) and a._fused_decode_ok(h, cache)
-                and _fused_ok(*(n.weight for n in norms), *(x.weight for x in lins))
-                and all(_dec_weight_ok(h.shape[0], x.weight) for x in (a.q_proj, a.o_proj, m.up_proj, m.down_proj)))
+                and _fused_ok(*(n.weight for n in norms), *(x.weight for x in lins)))
 
     def _decode_step(self, h, cache: LogoKVCache, position_embeddings, position_ids):
         """One decode step of ``h [B, 1, C]``: the same arithmetic as ``forward``,
-        each projection one launch with the norm, residual add or SwiGLU
-        beside it."""
-        a, n1, n2 = self.self_attn, self.input_layernorm, self.post_attention_layernorm
-        qkv = dec_linear(h, a._decode_weight(), norm_w=n1.weight, eps=n1.variance_epsilon)
+        each projection with the norm, residual add or SwiGLU beside it."""
+        a = self.self_attn
+        qkv = rows_product(h, a._decode_weight(), norm=self.input_layernorm)
         out, _ = a._decode_rows(qkv, cache, position_embeddings, position_ids)
-        h = dec_linear(out, a.o_proj.weight, resid=h)
-        act = dec_linear(h, self.mlp._gate_up_weight(), norm_w=n2.weight, eps=n2.variance_epsilon, glu=True)
-        return dec_linear(act, self.mlp.down_proj.weight, resid=h)
+        h = rows_product(out, a.o_proj.weight, resid=h)
+        act = rows_product(h, self.mlp._gate_up_weight(), norm=self.post_attention_layernorm, glu=True)
+        return rows_product(act, self.mlp.down_proj.weight, resid=h)
 
     def forward(self, hidden_states, attention_mask=None, position_ids=None, cu_seqlens=None,
                 past_key_value: Optional[LogoKVCache] = None, position_embeddings=None):

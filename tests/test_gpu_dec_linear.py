@@ -140,3 +140,28 @@ def test_weights_of_a_tensor_subclass_keep_their_arithmetic(gpu):
         want = 2 * torch.nn.functional.linear(x, lin.weight)
         lin.weight = torch.nn.Parameter(lin.weight.detach().as_subclass(_Scaled), requires_grad=False)
         assert torch.equal(linear_rows(lin, x), want)
+
+
+def test_a_stacked_weight_past_the_kernels_size(gpu):
+    """gate and up of 2^29 elements each, which stacked are one more than the
+    kernel takes: the step takes the library's product there."""
+    from logo_amd.layers import LoGoConfig, rope_cos_sin
+    from logo_amd.model import LoGoDecoderLayer
+    from logo_amd.ops.decode import LogoKVCache
+
+    cfg = LoGoConfig(hidden_size=4096, num_attention_heads=32, num_key_value_heads=4, num_hidden_layers=1,
+                     intermediate_size=131072, gate_thres_init=-1.0)
+    with torch.device(gpu):
+        torch.manual_seed(0)
+        layer = LoGoDecoderLayer(cfg, 0).to(torch.bfloat16).eval()
+    cache = LogoKVCache(1, 2, 4, 128, 32, window=128, device=gpu)
+    cache.set_length(5)
+    h = torch.randn(2, 1, 4096, device=gpu).bfloat16()
+    pe = rope_cos_sin(cache.positions(1), 128, cfg.rope_theta, torch.bfloat16)
+    with torch.no_grad():
+        assert layer._decode_ok(h, cache)
+        got = layer._decode_step(h, cache, pe, None).double()
+        want = layer(h, past_key_value=cache, position_embeddings=pe).double()
+    assert float((got - want).norm() / want.norm()) <= 2e-2
+    del layer, cache
+    torch.cuda.empty_cache()
