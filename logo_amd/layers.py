@@ -29,8 +29,8 @@ import torch.nn.functional as F
 
 from .ops.decode import LogoKVCache, decode_attn, decode_attn_fused, decode_qkv
 from .ops.epilogue import logo_epilogue
-from .ops.glue import (attn_inputs, dec_linear, dec_linear_ok, global_maps_, global_maps_ok, head_linear, head_proj,
-                       rms_norm, rope, rope_apply_, silu_mul)
+from .ops.glue import (attn_inputs, dec_linear, dec_linear_faster, dec_linear_ok, global_maps_, global_maps_ok,
+                       head_linear, head_proj, rms_norm, rope, rope_apply_, silu_mul)
 from .ops.sq_attn import dense_causal_attn, sq_full_attn, swa_attn
 
 __all__ = ["LoGoConfig", "LoGoAttention", "Attention", "RMSNorm", "rope_cos_sin", "apply_rope", "position_ids_for"]
@@ -146,8 +146,9 @@ def rows_product(x, w, norm=None, resid=None, glu=False):
 
 def linear_rows(lin: nn.Linear, x):
     """``lin(x)``, on ``dec_linear`` for the few rows of a decode step."""
-    if 0 < x.numel() <= 16 * x.shape[-1] and _plain(lin) and type(lin) is nn.Linear and lin.bias is None \
-            and _fused_ok(x, lin.weight):
+    k = x.shape[-1]
+    if 0 < x.numel() <= 16 * k and _plain(lin) and type(lin) is nn.Linear and lin.bias is None \
+            and _fused_ok(x, lin.weight) and dec_linear_faster(x.numel() // k, lin.weight.shape[0], k):
         return rows_product(x, lin.weight)
     return lin(x)
 
@@ -421,7 +422,9 @@ class LoGoAttention(nn.Module):
         """Decode step with the stacked q / k / v / gate GEMM and one launch for
         the global projections, RoPE and cache appends (same arithmetic as the
         step-by-step path: the same roundings, in the same order)."""
-        qkv = rows_product(hidden_states, self._decode_weight())
+        w = self._decode_weight()
+        faster = dec_linear_faster(hidden_states.shape[0], *w.shape)
+        qkv = rows_product(hidden_states, w) if faster else F.linear(hidden_states, w)
         return self._decode_rows(qkv, cache, position_embeddings, position_ids)
 
     def _decode_rows(self, qkv, cache: LogoKVCache, position_embeddings, position_ids):

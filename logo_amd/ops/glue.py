@@ -15,7 +15,7 @@ import torch.nn.functional as F
 from .. import _lib
 
 __all__ = ["rope_apply_", "rope", "RopeFunction", "rms_norm", "head_proj", "add_rms_norm", "silu_mul",
-           "dec_linear", "dec_linear_ok", "head_linear", "HeadLinearFunction", "head_linear_grad_acc",
+           "dec_linear", "dec_linear_ok", "dec_linear_faster", "head_linear", "HeadLinearFunction", "head_linear_grad_acc",
            "global_maps_", "global_maps_ok", "attn_inputs", "AttnInputsFunction"]
 
 
@@ -193,6 +193,41 @@ def dec_linear_ok(rows: int, w) -> bool:
     2048: 12.5 against 19.6 us for N = 6152)."""
     return (0 < rows <= DEC_LINEAR_MAX_ROWS and w.dim() == 2 and w.shape[1] % 32 == 0 and w.is_contiguous()
             and w.data_ptr() % 16 == 0 and w.numel() < 1 << 30)
+
+
+def dec_linear_faster(rows: int, n: int, k: int) -> bool:
+    """Whether ``dec_linear`` takes a product with nothing beside it (a LM head, a
+    projection by itself) in less time than the library's GEMM.  In a decoder
+    layer it does for every size up to 16 rows, by the launches that it spares.
+
+    Up to K = 2048 a wave's part of K is one batch of copies and a CU holds two
+    workgroups of 16 weight rows; every one of them reads all of x, which counts
+    where there are many.  Beyond, a workgroup takes a CU's LDS and waits for its
+    batches in turn, so the kernel wins while one round of workgroups holds N.
+    Replayed back to back from a graph over weights larger than the caches, kernel
+    / library in us:
+
+    ==============  ===============  ===============  ===============
+    N x K           4 rows           12 rows          16 rows
+    ==============  ===============  ===============  ===============
+    6144 x 2048     7.9 / 12.6       9.6 / 12.5       10.2 / 12.4
+    32000 x 1024    12.5 / 19.0      14.3 / 17.3      16.1 / 17.4
+    32000 x 2048    26.3 / 33.1      30.0 / 33.2      33.0 / 31.4
+    128256 x 1536   66.2 / 76.9      79.9 / 78.0      88.4 / 77.3
+    4096 x 3072     7.6 / 12.8       8.1 / 12.8       8.5 / 12.7
+    5120 x 3072     11.9 / 11.6      13.2 / 11.6      14.3 / 11.6
+    32000 x 3072    46.7 / 43.6      51.9 / 44.1      55.8 / 42.6
+    32000 x 4096    57.3 / 60.9      64.0 / 61.2      68.4 / 60.5
+    128256 x 4096   201 / 188        228 / 186        251 / 186
+    ==============  ===============  ===============  ===============
+
+    Behind other kernels the library's GEMM takes 10 to 30 us more than that, so
+    up to 4 rows stay here for K > 2048 too: a decode step of three layers and a
+    128256 x 3072 head 498 against 515 us at one row, 530 / 535 at four, 566 / 557
+    at eight, 663 / 621 at sixteen."""
+    if k <= 2048:
+        return n <= 8192 or (rows * k <= 12 * 2048 if n <= 65536 else rows <= 10)
+    return k <= 4096 and (n <= 4096 or rows <= 4)
 
 
 def _aligned16(t):

@@ -54,6 +54,21 @@ def test_dec_linear(gpu, m, n, k, mode):
     assert bool(((got - ref).abs() <= tol).all()), f"max excess {float(((got - ref).abs() - tol).max()):.3e}"
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 64, 256), (16, 8193, 2048), (12, 8193, 2048), (4, 4097, 2080), (5, 4097, 2080), (1, 40, 4128)])
+def test_single_products_on_both_sides_of_the_rule(gpu, m, n, k):
+    """On the kernel or the library's product: a bf16 rounding from float64."""
+    from logo_amd.layers import linear_rows
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, 1, k, generator=g).bfloat16().to(gpu)
+    lin = torch.nn.Linear(k, n, bias=False).to(device=gpu, dtype=torch.bfloat16)
+    with torch.no_grad():
+        got = linear_rows(lin, x).double()
+    ref = x.double() @ lin.weight.detach().double().T
+    assert got.shape == ref.shape
+    assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5).all())
+
+
 def test_hooks_and_other_modules_keep_their_calls(gpu):
     """A decode step calls a module that carries a forward hook (or is no plain
     linear layer) as before, with the same logits within bf16 rounding."""
