@@ -439,7 +439,7 @@ int logo_head_linear_grad_acc(const void* dy, int64_t lddy, const void* w, const
  *   xr_i = rope(x_i), y_i = rope(x_i W_i)   where xr_i is not null (it may be x_i),
  *   y_i = x_i W_i                           where it is.
  * w_i [h_i, d, d]; cos / sin [n_tokens, d] (may be null if no xr_i is given).
- * Unused x_i are null.  All pointers 16-byte aligned.
+ * Unused x_i are null.  At least one token.  All pointers 16-byte aligned.
  */
 int logo_global_maps(const void* x0, const void* w0, void* xr0, void* y0, int h0, const void* x1, const void* w1,
                      void* xr1, void* y1, int h1, const void* x2, const void* w2, void* xr2, void* y2, int h2,

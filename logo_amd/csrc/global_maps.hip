@@ -455,7 +455,8 @@ using namespace logo;
 
 static int gm_check(const void* cos, const void* sin, bool rope, int64_t n_tokens, int dtype) {
   LOGO_REQUIRE(dtype == LOGO_DTYPE_BF16, "only bf16 tensors are supported");
-  LOGO_REQUIRE(n_tokens >= 0 && n_tokens < ((int64_t)1 << 31), "n_tokens must be in [0, 2^31)");
+  // (no tokens: the weight gradients asked for would not be written)
+  LOGO_REQUIRE(n_tokens >= 1 && n_tokens < ((int64_t)1 << 31), "n_tokens must be in [1, 2^31)");
   LOGO_REQUIRE(!rope || (cos && sin), "null cos / sin");
   LOGO_REQUIRE(((uintptr_t)cos | (uintptr_t)sin) % 16 == 0, "cos and sin must be 16-byte aligned");
   return LOGO_OK;
@@ -494,7 +495,7 @@ extern "C" int logo_global_maps(const void* x0, const void* w0, void* xr0, void*
     t.heads = hs[i];
     heads += hs[i];
   }
-  if (heads == 0 || n_tokens == 0) return LOGO_OK;
+  if (heads == 0) return LOGO_OK;
   a.cos = static_cast<const bf16*>(cos);
   a.sin = static_cast<const bf16*>(sin);
   a.n = n_tokens;
@@ -547,7 +548,7 @@ extern "C" int logo_global_maps_bwd(const void* x0, const void* w0, const void* 
     any_dw |= dws[i] != nullptr;
   }
   LOGO_REQUIRE(!any_dw || (workspace && (uintptr_t)workspace % 16 == 0), "workspace must be 16-byte aligned memory");
-  if (heads == 0 || n_tokens == 0) return LOGO_OK;
+  if (heads == 0) return LOGO_OK;
   a.cos = static_cast<const bf16*>(cos);
   a.sin = static_cast<const bf16*>(sin);
   a.lddx = lddx;

@@ -98,6 +98,20 @@ def test_head_linear_grad_acc_rejects_bad_arguments():
         assert msg in lib.logo_last_error().decode()
 
 
+def test_global_maps_refuse_a_call_without_tokens():
+    """As the kernels they stand for: the weight gradients of no tokens would stay
+    unwritten (pointers are placeholders, empty tensors have null ones)."""
+    lib = _lib.lib()
+    p = ctypes.c_void_p(256)
+    for x in (p, None):
+        fwd = [x, p, None, x, 2] * 3
+        bwd = [x, p, x, x, x, p, 2, 0] * 3
+        assert lib.logo_global_maps(*fwd, p, p, 0, 128, _lib.DTYPE_BF16, None) == 1
+        assert "n_tokens" in lib.logo_last_error().decode()
+        assert lib.logo_global_maps_bwd(*bwd, p, p, 1024, p, 0, 128, _lib.DTYPE_BF16, None) == 1
+        assert "n_tokens" in lib.logo_last_error().decode()
+
+
 def test_read_calibration_rejects_bad_arguments():
     """The streaming-read calibration refuses null pointers, an unaligned
     buffer or size and grids outside [1, 65536], for either load kind, before

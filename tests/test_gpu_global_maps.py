@@ -91,3 +91,13 @@ def test_layouts_that_are_not_the_kernels(gpu):
     assert shifted[0].data_ptr() % 16 and _aligned16(shifted[0]).data_ptr() % 16 == 0
     for a, b in zip(attn_inputs(h, *lin, ws, *shifted, 2, 2), ref):
         assert torch.equal(a, b)
+
+
+def test_no_tokens_are_refused(gpu):
+    """An empty batch is an error, not uninitialised weight gradients."""
+    _, ws, _, _, _ = _inputs(1, 2, 2, 128, 4)
+    lin = [torch.nn.Linear(256, k, bias=False).cuda().bfloat16() for k in (256, 256, 256, 1)]
+    h = torch.empty(1, 0, 256, dtype=torch.bfloat16, device="cuda")
+    cos = torch.empty(1, 0, 128, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(RuntimeError, match="n_tokens"):
+        attn_inputs(h, *lin, [w.requires_grad_() for w in ws], cos, cos.clone(), 2, 2)
