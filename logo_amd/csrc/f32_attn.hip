@@ -15,9 +15,9 @@
 //             dV, wave B dP, dS and dK, P passing through LDS.  (One wave per 16
 //             keys with both accumulators needs 230 registers at D = 128, two
 //             waves a SIMD.)
-// RW / KG and NP / RG follow from the size of the call (f32_split).
-// All partial sums are added in a fixed order.  exp2 is the hardware's (results
-// below 2^-126 are zero).
+// RW / KG and NP / RG follow from the size of the call (dispatch_rows,
+// dispatch_dkv).
+// All partial sums are added in a fixed order.
 // Measured against 16 rows or keys a wave, 64 a workgroup, no key or row groups:
 // T = 4096, 16 heads, D = 128, a quarter of the rows, forward + backward 1255 ->
 // 750 us (MFMA busy 55 / 65 / 67% in forward / dq / dk/dv); 512 tokens, 4 heads,
@@ -55,6 +55,22 @@ __device__ __forceinline__ float swap16_sum(float x) {
 }
 __device__ __forceinline__ float col_max(float x) { return pair_max(swap16_max(x)); }
 __device__ __forceinline__ float col_sum(float x) { return pair_sum(swap16_sum(x)); }
+
+// exp2 of four scores.  The hardware's exp2 flushes results below 2^-126, where a
+// probability still gives a gradient if dO v is large, so a wave with a score
+// there takes exp2f (whose other results are the hardware's).  At T = 4096, 16
+// heads, D = 128, a quarter of the rows, forward + backward 792 us with the
+// hardware's exp2, 802 so, 814 with exp2f in every wave.
+__device__ __forceinline__ f32x4 exp2_4(f32x4 x) {
+  if (__ballot(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])) < -126.f)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = exp2f(x[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = fast_exp2(x[j]);
+  }
+  return x;
+}
 
 __device__ __forceinline__ void barrier_all() {
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -263,10 +279,12 @@ __global__ __launch_bounds__(64 * kWaves) void f32_rows_kernel(const AttnArgs a)
         }
       }
 #pragma unroll
+      for (int j = 0; j < 4; ++j) s[j] = fmaf(s[j], c, -lse);
+      s = exp2_4(s);
+#pragma unroll
       for (int j = 0; j < 4; ++j) {
-        float pr = fast_exp2(fmaf(s[j], c, -lse));
-        if (mask && kt + 4 * G + j > p) pr = 0.f;
-        s[j] = pr * (dp[j] - dlt);
+        if (mask && kt + 4 * G + j > p) s[j] = 0.f;
+        s[j] *= dp[j] - dlt;
       }
       tr_product<D>(tl, kb, s, acc);
     } else {
@@ -278,9 +296,10 @@ __global__ __launch_bounds__(64 * kWaves) void f32_rows_kernel(const AttnArgs a)
       const float m_new = fmaxf(m_run, col_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
       // a query that has seen no key keeps m = -inf, P and l zero through base 0
       const float base = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = fast_exp2(m_run - base);
+      const float alpha = exp2f(m_run - base);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] = fast_exp2(s[j] - base);
+      for (int j = 0; j < 4; ++j) s[j] -= base;
+      s = exp2_4(s);
       l_run = l_run * alpha + ((s[0] + s[1]) + (s[2] + s[3]));
       m_run = m_new;
       if (__ballot(alpha != 1.f)) {
@@ -476,10 +495,10 @@ __global__ __launch_bounds__(64 * kWaves) void f32_dkv_kernel(const AttnArgs a) 
           const int4 p4 = lds_load(reinterpret_cast<const int4*>(st + 2 * KT + 4 * G));
           const int pq[4] = {p4.x, p4.y, p4.z, p4.w};
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float pr = fast_exp2(fmaf(x[j], c, -l4[j]));
-            x[j] = valid_k && key <= pq[j] ? pr : 0.f;
-          }
+          for (int j = 0; j < 4; ++j) x[j] = fmaf(x[j], c, -l4[j]);
+          x = exp2_4(x);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) x[j] = valid_k && key <= pq[j] ? x[j] : 0.f;
           pbuf[(t & 1) * 64 + l] = x;
         }
       }

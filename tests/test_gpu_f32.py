@@ -57,3 +57,34 @@ def test_tile_edges_every_row_selected(gpu, lens, d):
 ])
 def test_waves_of_a_workgroup(gpu, lens, hq, h, d, rows, per_head):
     _check(gpu, lens, hq, h, d, rows, per_head)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_probabilities_below_the_normal_range_count(gpu, d):
+    """Key 0 has probability 2^-131 to 2^-135 in every later row, a subnormal fp32
+    number, and dO v_0 = 2^60: its share of dq and all of dk_0 come from their
+    product, which fp32 holds.  A subnormal of 15 bits or more and scores of 135
+    with a few 2^-24 of relative error leave 1e-4."""
+    from logo_amd.ops import sq_full_attn
+
+    n = 40
+    q, k, v, do = (torch.zeros(n, 2, d) for _ in range(4))
+    q[:, :, 0] = 8.0
+    k[0, :, 0] = -130.0 / 8.0
+    v[0, :, 1] = 2.0 ** 30
+    do[1:, :, 1] = 2.0 ** 30
+    do[:, :, 2] = torch.randn(n, 2, generator=gen(5))
+    v[1:, :, 2] = torch.randn(n - 1, 2, generator=gen(6))
+    scale = float(np.log(2.0))  # scores in the log2 domain: 8 times k_0
+    sel = torch.ones(n, dtype=torch.bool)
+    cu = torch.tensor([0, n], dtype=torch.int32)
+    qg, kg, vg = (x.to(gpu)[None].requires_grad_() for x in (q, k, v))
+    o = sq_full_attn(qg, kg, vg, sel.to(gpu)[None], cu_seqlens=cu.to(gpu), scale=scale)
+    _, dk, dv = torch.autograd.grad(o, (qg, kg, vg), do.to(gpu)[None])
+    qn, kn, vn, dn = (x.double().numpy() for x in (q, k, v, do))
+    ro, _ = attn.sq_attn_fwd(qn, kn, vn, sel.numpy(), cu.numpy(), scale=scale)
+    _, rdk, rdv = attn.sq_attn_bwd(qn, kn, vn, ro, dn, sel.numpy(), cu.numpy(), scale=scale)
+    want = rdk[0, :, 0]
+    assert 0 < np.abs(want).max() < 2.0 ** -50
+    got = dk[0, 0, :, 0].double().cpu().numpy()
+    assert np.abs(got - want).max() <= 1e-4 * np.abs(want).max(), (got, want)
