@@ -1,7 +1,11 @@
-"""GPU parity of the generic attention kernels (logo_amd/csrc/gen_attn.hip):
-fp32 inputs computed in fp32, and head dims in (128, 256].
+"""GPU parity of fp32 inputs computed in fp32, and of head dims in (128, 256].
 
-* fp32 (BASELINE config 1: B=1, H=4, T=512, D=64, N(0, 1) inputs, Bernoulli
+Without a window they run on kernels of their own (logo_amd/csrc/f32_attn.hip,
+wide_attn.hip) while q is below 4 GB, with a window or from there on on the
+generic ones (gen_attn.hip): here those of head dim 256 with a window;
+tests/test_gpu_over_4gb.py has the others.
+
+* fp32 (B=1, H=4, T=512, D=64, N(0, 1) inputs, Bernoulli
   0.5 selection), plus GQA, packed segments, the per-head extension, D=128 and
   D=256, and mixed fp32 / bf16 inputs (widened to fp32).  The reference's dots
   run in the input dtype with P kept in fp32 for PV
@@ -12,8 +16,8 @@ fp32 inputs computed in fp32, and head dims in (128, 256].
   kernels on the same inputs rounded to bf16.
 * K, V in (128, 256], V != K, GQA, in bf16 and fp16, on the query-sparse path
   (the reference takes any K <= 256 in one block, :344), and the dense and
-  sliding-window branches at D=256 in bf16: the north-star bound (max-abs
-  2e-2, mean-abs 2e-3) against the float64 oracle, unselected rows zero.
+  sliding-window branches at D=256 in bf16: max-abs 2e-2 and
+  mean-abs 2e-3 against the float64 oracle, unselected rows zero.
 """
 
 import numpy as np
@@ -135,7 +139,7 @@ def test_dense_and_window_branches_at_d256(gpu, window):
 
 @pytest.mark.parametrize("dtype,d", [(torch.float32, 64), (torch.bfloat16, 256)])
 def test_generic_zero_rows_and_empty_lanes(gpu, dtype, d):
-    """The generic kernels' zero rows: an empty selection (every output and
+    """Zero rows of fp32 and D = 256: an empty selection (every output and
     gradient exactly zero except dk / dv, which are zero too since no row
     sees any key), and a per-head selection where one head has no rows and
     another one row, over packed segments with an empty one; against the

@@ -2,7 +2,8 @@
 with q below 4 GB they run on kernels that address its rows by 32 bits
 (logo_amd/csrc/wide_attn.hip, f32_attn.hip), from there on on the generic ones
 (gen_attn.hip).  Packed segments of every tile remainder at both ends of the
-tensors, GQA, one selection or one per head, dense rows; the first and the last
+tensors, GQA, one selection or one per head (one head without rows, one with a
+single one), dense rows; the first and the last
 segments against the float64 oracle, with the bounds of the kernels' own tests,
 and every unselected row zero."""
 
@@ -40,6 +41,9 @@ def test_first_and_last_segments(gpu, side, dtype, d, rows, per_head):
     g = torch.Generator(device=gpu).manual_seed(d)
     q, k, v, do = (torch.empty(n, x, d, dtype=dtype, device=gpu).normal_(generator=g) for x in (HQ, H, H, HQ))
     sel = None if rows is None else torch.rand((n, HQ) if per_head else (n,), generator=g, device=gpu) < rows
+    if per_head:
+        sel[:, 1:3] = False
+        sel[n - 5, 2] = True
     for x in (q, k, v):
         x.requires_grad_()
     print(f"{side} 4 GB: {dtype} d={d} n={n}", flush=True)
