@@ -23,7 +23,7 @@ def test_header_symbols_are_exported():
 def test_abi_version_and_workspace():
     lib = _lib.lib()
     assert lib.logo_abi_version() == 7
-    # the generic kernels serve d = 256 and fp32; they never split
+    # d = 256 and fp32 read q and dO in place; their split, at d = 256 in 16 bits, has a size function of its own
     assert [lib.logo_sq_generic(d, t) for d in (64, 128, 256) for t in (_lib.DTYPE_BF16, _lib.DTYPE_F16)] == \
         [0, 0, 0, 0, 1, 1]
     assert all(lib.logo_sq_generic(d, _lib.DTYPE_F32) == 1 for d in (64, 128, 256))
