@@ -160,8 +160,9 @@ __global__ __launch_bounds__(64 * kDlWaves) void dec_linear_kernel(const DecLinA
   for (int bt = 0; bt < nb; ++bt) {
     const int s0 = s_lo + U * bt, ns = min(U, s_hi - s0);
     if (bt > 0) load_x(s0, ns);
-    // this batch's copies have landed; the next batch's may be in flight
-    // (they were issued after x of batch 0 and before x of this one)
+    // all copies have landed, this batch's and the next one's: past the first
+    // batch, x of this one was loaded behind them, and loads return in order.  So
+    // a range of three batches (K = 5632) copies two, computes, copies the third
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const char* t = tile + (bt & 1) * TL::BYTES;
 #pragma unroll

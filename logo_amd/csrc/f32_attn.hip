@@ -19,10 +19,12 @@
 // dispatch_dkv).
 // All partial sums are added in a fixed order.
 // Measured against 16 rows or keys a wave, 64 a workgroup, no key or row groups:
-// T = 4096, 16 heads, D = 128, a quarter of the rows, forward + backward 1255 ->
-// 750 us (MFMA busy 55 / 65 / 67% in forward / dq / dk/dv); 512 tokens, 4 heads,
-// D = 64: the three kernels 34 + 42 + 37 -> 13 + 13 + 13 us.  Running S of the
-// next tile beside the softmax of the current one measured no faster.
+// T = 4096, 16 heads, D = 128, a quarter of the rows, forward + backward 1238 to
+// 1306 -> 715 to 802 us on the boxes measured; 512 tokens, 4 heads, D = 64: the
+// three kernels 34 + 42 + 36 -> 13 + 13 + 12 us.  At T = 8192 the matrix units are
+// 54 / 75 / 79% busy (forward, dq, dk/dv); the forward's waves meet at a barrier
+// every 16 keys and do their softmax together.  Running S of the next tile beside
+// the softmax of the current one measured no faster.
 #include "sq_attn.hpp"
 
 #include <algorithm>

@@ -21,7 +21,7 @@
 // scale * log2(e) in fp32 (:93); P and dS are rounded to the input type
 // before their products (:99, :206-207), which for fp32 means no rounding.
 //
-// Structure (simple, one LDS buffer, no software pipelining):
+// Structure (simple, two LDS stages, no software pipelining):
 //   16x16 MFMA tiles with a 16-deep k step for every element type:
 //   v_mfma_f32_16x16x16_bf16 / _f16 (one per k step) and
 //   v_mfma_f32_16x16x4_f32 (four per k step).  Lane l = 16 G + i holds

@@ -509,9 +509,11 @@ bool swa_bwd_applies(const AttnArgs& a, bool sparse, bool half);
 int swa_launch_bwd(const AttnArgs& a, hipStream_t st, int d);
 
 // The generic kernels (gen_attn.hip): head dim 256 (bf16, and fp16 in sparse
-// mode) and fp32 in sparse mode (d = 64, 128, 256).  gen_applies: whether a
-// call with head dim d and element type dtype runs on them (the entry points
-// route such calls there before any tuned kernel).
+// mode) and fp32 in sparse mode (d = 64, 128, 256), where the families below do
+// not serve the call: a window, or q of 4 GB and more.  gen_applies: whether head
+// dim d and element type dtype belong to these kernels and those families, which
+// read q and dO in place (the entry points route such calls there before any
+// tuned kernel).
 bool gen_applies(int d, int dtype);
 int gen_launch_fwd(const AttnArgs& a, hipStream_t st, int d, int dtype, bool sparse);
 int gen_launch_delta(const AttnArgs& a, hipStream_t st, int d, int dtype, bool sparse);

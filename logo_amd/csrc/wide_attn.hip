@@ -10,17 +10,23 @@
 //   dk/dv   : two pairs of waves x 32 keys; in a pair one wave computes S, P
 //             and dV, the other dP, dS and dK, P passing through LDS; 32
 //             gathered rows of q and dO a step.
-// Bound: MFMA issue.  An operand read from LDS feeds one MFMA here (the wave's
-// registers hold no second row block), 1 KB per 32 cycles and SIMD: all of the
-// LDS bandwidth at the MFMA peak, so about half of that peak is the aim.
-// Measured at T = 8192, 16 heads, a quarter of the rows, forward + backward:
-// 822 us, 1834 on the generic kernels (16 rows or keys a wave on 16x16 MFMAs,
-// one LDS operand read per half as many FLOPs, no pipelining); 4001 tokens, 4
-// heads, forward only with split key ranges: 70 against 227 us; a few hundred
-// tokens are bound by the launches either way.
-// Numerics are the generic kernels': S from the unscaled inputs, scaled in
-// fp32; P and dS rounded to the input type; the dP accumulators start from
-// -delta.  q and dO rows are gathered in place (no compacted copies).
+// An operand read from LDS feeds one MFMA here (the wave's registers hold no
+// second row block), 1 KB per 32 cycles and SIMD: all of the LDS bandwidth at the
+// MFMA peak, so about half of that peak is the most this form can reach.
+// Bound: waits.  One wave a SIMD is resident; at T = 8192, 16 heads, a quarter of
+// the rows it waits 40 / 33 / 34% of its time (forward, dq, dk/dv: for barriers,
+// the copies behind them, LDS operands) with the matrix units 26 / 37 / 32%, the
+// VALU 20 / 16 / 25% and the LDS 13 / 19 / 22% busy.  Forward + backward there:
+// 806 to 897 us on the boxes measured, 1834 to 1866 on the generic kernels (16
+// rows or keys a wave on 16x16 MFMAs, one LDS operand read per half as many FLOPs,
+// no pipelining); 4001 tokens, 4 heads, forward only with split key ranges: 70
+// against 227 us; a few hundred tokens are bound by the launches either way.
+// Numerics are the generic kernels' but for three things: S from the unscaled
+// inputs, scaled in fp32; P and dS rounded to the input type.  The dP accumulators
+// start from -delta; the forward's running maximum may lag by up to 2^8 (o is
+// 0.05% further from float64 so, relative to its error of 1.9e-3; dq, dk and dv as
+// near); the hardware's exp2 flushes P below 2^-126, as in the kernels of dim 64
+// and 128.  q and dO rows are gathered in place (no compacted copies).
 #include "sq_attn.hpp"
 
 #include <algorithm>
