@@ -129,28 +129,31 @@ inline void split_setup(AttnArgs& a, int wgs_per_cu, size_t floats) {
 constexpr int kDkvRows = 128;
 
 // Fewest steps of a piece of a dk/dv key block, where a kv head has nt of them
-// and cap is two workgroups a CU (one CU holds one).  A piece starts like a
-// block (8 to 10 us with the loads of K and V) and writes 128 KB of partials at
-// D = 128, so pieces pay while CUs are idle; beyond one block a CU they have to
-// be long enough to make up for a second round.  A block with fewer than two
-// times these steps is left whole.  dk/dv alone, cut against whole, D = 64 and
-// 128, 2 to 16 kv heads, 500 to 24000 tokens, one and six segments:
-//   blocks below half the CUs (3): 6 to 11 steps in the heaviest block 0.78x,
-//     12 to 25 0.52x, 64 and more 0.35x
-//   up to one a CU (16): 26 to 39 steps 0.80x, 64 and more 0.75x; cut into pieces
-//     of 5 steps, 12 to 17 steps took up to 1.24x
-//   up to 9/8 of them (24): 64 to 99 steps 0.91x, from 100 on 0.73x
-//   up to 3/2 (96): from 176 steps on 0.90x; pieces of 24 steps up to 1.23x
+// and cap is two workgroups a CU (one CU holds one), and fewest steps that a
+// segment's first block has if its blocks are cut.  A piece starts like a block (8
+// to 10 us with the loads of K and V) and writes 128 KB of partials at D = 128, so
+// pieces pay while CUs are idle; beyond, they have to be long enough to make up for
+// a second round.  dk/dv alone, cut against whole, D = 64 and 128, 1 to 16 kv heads,
+// 1000 to 24000 tokens, one and six segments:
+//   blocks below half the CUs (3): 6 to 11 steps in the heaviest block 0.81x,
+//     12 to 25 0.55x, 64 and more 0.32x
+//   up to one a CU (10): 18 to 39 steps 0.85x, 64 and more 0.54x; in pieces of 5
+//     steps, 12 to 17 steps took up to 1.27x
+//   up to 9/8 of them (16): 40 to 99 steps 0.85x, from 100 on 0.70x; in pieces of 8,
+//     12 to 17 steps up to 1.26x
+//   up to 3/2 (24): from 192 steps on 0.87x; below 144, where only the first blocks
+//     reach two pieces, up to 1.20x
 constexpr int dkv_min_steps(int nt, int cap) {
-  return 4 * nt < cap ? 3 : 2 * nt <= cap ? 16 : 16 * nt <= 9 * cap ? 24 : 96;
+  return 4 * nt < cap ? 3 : 2 * nt <= cap ? 10 : 16 * nt <= 9 * cap ? 16 : 24;
 }
+constexpr int dkv_gate_steps(int nt, int cap) { return (16 * nt <= 9 * cap ? 2 : 6) * dkv_min_steps(nt, cap); }
 
 // Pieces per kv head that dk/dv aims for; 0 where no block of n tokens can be
 // cut: too many blocks, or too few steps with every row selected.
 inline int dkv_split_cap(int64_t n, int hq, int h) {
   const int cap = split_cap_for(h, 1);
   const int64_t nt = (n + kBKV - 1) / kBKV, steps = hq / h * ((n + kDkvRows - 1) / kDkvRows);
-  return cap >= 2 && 4 * nt <= 3 * (int64_t)cap && steps >= 2 * dkv_min_steps((int)nt, cap) ? cap : 0;
+  return cap >= 2 && 4 * nt <= 3 * (int64_t)cap && steps >= dkv_gate_steps((int)nt, cap) ? cap : 0;
 }
 
 // Most workgroups of a kv head over the block counts that n tokens in nseq

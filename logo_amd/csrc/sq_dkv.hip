@@ -41,14 +41,23 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
   const int ntk = meta0[2];
   const int nper = WINDOW ? 1 : split_pieces(ntk, a.split_cap);
   if (rank >= ntk * nper) return;
-  // early key blocks (most queries) first; the first pieces of all blocks ahead
-  // of the others, so that workgroups without a piece, where the blocks have too
-  // few steps, come when the others run
-  const int piece = rank / ntk;
-  const int tile = rank - piece * ntk;
-  const int min_steps = dkv_min_steps(ntk, a.split_cap);
+  const int min_steps = dkv_min_steps(ntk, a.split_cap), gate = dkv_gate_steps(ntk, a.split_cap);
   const int32_t* meta_h = meta0 + (int64_t)(a.lanes > 1 ? h * a.g : 0) * a.meta_stride;  // the group's first head
-  if (piece > 0 && (meta_h[0] + RS - 1) / RS * a.g < 2 * min_steps) return;
+  // Early key blocks (most queries) first.  Where half of an average segment's
+  // blocks have steps for all pieces, the pieces of a block together; else the
+  // first piece of every block, then the others of each block in turn, so that the
+  // workgroups without a piece come last (in between, at every second rank, they
+  // would leave the XCDs or shader engines whose turn they take without work).
+  const int rows = meta_h[0];
+  int tile = rank, piece = 0;
+  if ((rows / a.nseq + RS - 1) / RS * a.g >= 2 * nper * min_steps) {
+    tile = rank / nper;
+    piece = rank - tile * nper;
+  } else if (rank >= ntk) {
+    tile = (rank - ntk) / (nper - 1);
+    piece = rank - ntk - tile * (nper - 1) + 1;
+  }
+  if (piece > 0 && (rows + RS - 1) / RS * a.g < gate) return;
   const int32_t* cu_tk = meta0 + kMetaHdr + 2 * (a.nseq + 1);
   const int s = seg_of(cu_tk, a.nseq, tile);
   const int k0 = (tile - cu_tk[s]) * kBKV;
@@ -65,7 +74,10 @@ __global__ __launch_bounds__(256) LOGO_OCC_DKV void sq_dkv_kernel(const AttnArgs
   int nsplit = 1;
   if (nper > 1) {
     const int lo = meta_h[kMetaHdr + s], hi = meta_h[kMetaHdr + s + 1];
-    int total = (hi - lo + RS - 1) / RS * a.g;
+    // the block's steps if the rows were even over the segment, then, where they
+    // would be enough, its own
+    int total = ((int)((hi - lo) * (float)(seqlen - k0) / (float)seqlen) / RS + 1) * a.g;
+    if ((hi - lo + RS - 1) / RS * a.g < gate) total = 0;
     if (total >= 2 * min_steps) {
       const int r0 = SPARSE ? wave_lower_bound(row_view<SPARSE>(a, a.lanes > 1 ? h * a.g : 0, bos).ps, lo, hi, k0)
                             : min(lo + k0, hi);

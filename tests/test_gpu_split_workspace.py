@@ -72,16 +72,18 @@ def test_dq_and_dkv_share_a_workspace(gpu, n, hq, h, d, cu, dkv_splits):
     (4000, 4, 2, 64, 0.05, False, False),
     (2000, 16, 4, 128, 0.25, False, True),
     (2000, 16, 4, 64, 0.25, True, True),
-    # up to one a CU: from 32 steps on
-    (4000, 16, 8, 64, 0.4, False, False),
-    (4000, 32, 8, 64, 0.4, False, True),
+    # up to one a CU: from 20 steps on
+    (4000, 16, 8, 64, 0.2, False, False),
+    (4000, 16, 8, 64, 0.4, False, True),
     (6000, 16, 4, 128, 0.05, True, False),
-    # more: from 48, then 192 steps on
+    # more: from 32, then 144 steps on
     (9000, 16, 4, 64, 0.08, False, False),
     (9000, 16, 4, 64, 0.4, False, True),
     (6000, 32, 8, 64, 0.4, False, False),
+    (6000, 32, 8, 64, 0.9, False, True),
     # no choice of rows gives the steps
-    (2000, 16, 16, 64, 1.1, False, False),
+    (1000, 4, 4, 64, 0.6, False, False),
+    (1100, 16, 16, 64, 1.1, False, False),
 ])
 def test_key_blocks_of_few_steps_stay_whole(gpu, n, hq, h, d, rows, per_head, splits):
     """dk/dv cuts a key block (and writes partials) only where its steps pay for
