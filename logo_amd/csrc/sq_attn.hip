@@ -232,7 +232,8 @@ extern "C" int logo_sq_fwd(const void* q, const void* k, const void* v, void* o,
   const bool sparse = q_idx != nullptr;
   const bool win = window >= 0;
   if (f32_applies(a, d, dtype, sparse)) return f32_launch(a, as_stream(stream), kPhaseFwd, d);
-  if (wide_applies(a, d, dtype)) return wide_launch(a, as_stream(stream), kPhaseFwd, sparse, dtype == LOGO_DTYPE_F16);
+  if (wide_applies(a, d, dtype) && n_tokens >= (int64_t)LOGO_WIDE_FWD_MIN_TOKENS * nseq)
+    return wide_launch(a, as_stream(stream), kPhaseFwd, sparse, dtype == LOGO_DTYPE_F16);
   if (gen_applies(d, dtype)) return gen_launch_fwd(a, as_stream(stream), d, dtype, sparse);
   return sq_launch_fwd(a, as_stream(stream), d, sparse, win, dtype == LOGO_DTYPE_F16);
 }

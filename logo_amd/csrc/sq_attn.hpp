@@ -49,6 +49,9 @@ struct AttnArgs {
   float* part;
   int* cnt;
   int split_cap;
+  // fewest keys of a piece, where all pieces run at once and where they take turns
+  // on the CUs (0: the 64-key alignment alone)
+  int split_keys, split_keys_turns;
   // the caller's workspace (host side only: the launchers carve part / cnt
   // from it when it is large enough for their kernel's split_cap)
   void* ws;
@@ -373,7 +376,9 @@ struct QTile {
     if (nper > 1) {
       // 64-key-aligned chunks; nsplit <= nper pieces, none empty
       const int span = kv_hi - kv_lo;
-      const int chunk = (((span + nper - 1) / nper) + 63) & ~63;
+      const int least = 2 * nt * nper <= a.split_cap ? a.split_keys : a.split_keys_turns;
+      const int most = least > 0 ? max(1, min(nper, span / least)) : nper;
+      const int chunk = (((span + most - 1) / most) + 63) & ~63;
       nsplit = (span + chunk - 1) / chunk;
       if (piece >= nsplit) return false;
       kv_lo += piece * chunk;
@@ -532,7 +537,8 @@ int f32_launch(const AttnArgs& a, hipStream_t st, int phase, int d);
 
 // Head dim 256 in 16-bit types without a window (wide_attn.hip): whether it
 // serves a call (q and dO below 4 GB, as its gathered copies address them by 32
-// bits), its phases, and the workspace that lets its forward and dq split.
+// bits; the forward of segments of at least LOGO_WIDE_FWD_MIN_TOKENS on average),
+// its phases, and the workspace that lets its forward and dq split.
 bool wide_applies(const AttnArgs& a, int d, int dtype);
 size_t wide_workspace_bytes(int hq);
 int wide_launch(const AttnArgs& a, hipStream_t st, int phase, bool sparse, bool half);

@@ -125,14 +125,15 @@ bool generic_path(const at::Tensor& q, int dtype) { return logo_sq_generic((int)
 // and tests that compare kernel variants bit for bit).
 constexpr size_t kMaxCachedStreams = 16;
 
-at::Tensor split_workspace(const at::Tensor& q, const at::Tensor& k, const at::Tensor& cu, int dtype) {
+at::Tensor split_workspace(const at::Tensor& q, const at::Tensor& k, const at::Tensor& cu, int dtype, bool fwd) {
   const char* env = std::getenv("LOGO_SQ_SPLIT");
   size_t bytes = 0;
   if (env == nullptr || env[0] != '0') {
     if (!generic_path(q, dtype))
       bytes = logo_sq_kv_workspace_bytes(q.size(0), (int)cu.numel() - 1, (int)q.size(1), (int)k.size(1),
                                          (int)q.size(2));
-    else if (dtype != LOGO_DTYPE_F32)
+    else if (dtype != LOGO_DTYPE_F32 && q.size(0) >= 2 * LOGO_WIDE_SPLIT_KEYS &&
+             !(fwd && q.size(0) < LOGO_WIDE_FWD_MIN_TOKENS * (cu.numel() - 1)))
       bytes = logo_sq_wide_workspace_bytes((int)q.size(1));
   }
   if (bytes == 0) return at::empty({0}, q.options().dtype(at::kByte));
@@ -172,7 +173,7 @@ std::tuple<at::Tensor, at::Tensor> sq_fwd(const at::Tensor& q, const at::Tensor&
   // tokens and for lse rows past each lane's rows, by the kernel).
   auto o = at::empty_like(q);
   auto lse = at::empty({hq, n}, q.options().dtype(at::kFloat));
-  auto ws = window < 0 ? split_workspace(q, k, cu, dtype) : at::empty({0}, q.options().dtype(at::kByte));
+  auto ws = window < 0 ? split_workspace(q, k, cu, dtype, true) : at::empty({0}, q.options().dtype(at::kByte));
   ok(logo_sq_fwd(cptr(q), cptr(k), cptr(v), mptr(o), lse.data_ptr<float>(), opt_ptr<int64_t>(q_idx),
                  opt_ptr<int32_t>(pos), meta.data_ptr<int32_t>(), cu.data_ptr<int32_t>(), n, (int)cu.numel() - 1,
                  (int)hq, (int)h, (int)d, (int)v.size(2), (int)lanes, (float)scale, (int)window, dtype,
@@ -209,7 +210,7 @@ struct Bwd {
     F fn = phase == 0 ? &logo_sq_bwd_delta : phase == 1 ? &logo_sq_bwd_dq : phase == 2 ? &logo_sq_bwd_dkv
                                                                                   : &logo_sq_bwd_dqkv;
     auto p = [](at::Tensor* t) -> void* { return t && t->numel() ? t->data_ptr() : nullptr; };
-    at::Tensor ws = phase >= 1 && window < 0 ? split_workspace(q, k, cu, dtype)
+    at::Tensor ws = phase >= 1 && window < 0 ? split_workspace(q, k, cu, dtype, false)
                                              : at::empty({0}, q.options().dtype(at::kByte));
     return fn(cptr(q), cptr(k), cptr(v), cptr(o), cptr(dout), lse.data_ptr<float>(),
               static_cast<float*>(p(delta)), p(q_sel), p(do_sel), p(dq), p(dk), p(dv), opt_ptr<int64_t>(q_idx),

@@ -55,6 +55,13 @@ def test_tile_edges_every_row_selected(gpu, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens", [[1], [31], [32], [33], [63, 65], [64, 1, 0, 127], [129], [160, 97]])
+def test_tile_edges_beside_a_long_segment(gpu, lens):
+    """(the forward of segments below 352 tokens on average is the generic one)"""
+    _check(gpu, [1900] + lens, 2, 1, 1.1)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("lens,hq,h,rows,per_head,dtype", [
     ([1500], 2, 2, 0.3, False, torch.bfloat16),       # rings and rounds of several steps, split key ranges
     ([700, 1, 650], 4, 1, 0.15, False, torch.bfloat16),
@@ -62,6 +69,9 @@ def test_tile_edges_every_row_selected(gpu, lens):
     ([513, 200], 2, 1, 0.4, False, torch.float16),
     ([300, 301], 2, 1, None, False, torch.bfloat16),  # dense rows
     ([1100], 8, 4, 0.02, False, torch.bfloat16),      # few rows
+    ([895], 2, 2, 0.6, False, torch.bfloat16),        # one key fewer than is cut, and the fewest that are
+    ([896, 5], 2, 2, 0.6, False, torch.bfloat16),
+    ([4500], 16, 16, 0.13, False, torch.bfloat16),    # pieces that take turns on the CUs
 ])
 def test_longer_sequences(gpu, lens, hq, h, rows, per_head, dtype):
     _check(gpu, lens, hq, h, rows, dtype, per_head)
