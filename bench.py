@@ -85,9 +85,9 @@ def parse():
     ap.add_argument("--swa", action="store_true",
                     help="run only the config-4 sliding-window (local branch) forward and "
                          "forward + backward measurement and print its result")
-    ap.add_argument("--generic", action="store_true",
-                    help="run only the generic-kernel measurement (head dim 256 in bf16, fp32 at D=128, "
-                         "config 1 in fp32) and print its result")
+    ap.add_argument("--wide-fp32", action="store_true",
+                    help="run only the measurement of head dim 256 in bf16 and of fp32 (at D=128, and "
+                         "512 tokens of D=64) and print its result")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="run one 1 GiB device-to-device copy before the workload (the reference kernel "
                          "for scaling rocprofv3 FETCH_SIZE / WRITE_SIZE counters to bytes)")
@@ -231,9 +231,9 @@ def swa_cfg4_measurement(q, k, v, do, iters=10):
             "bwd_of_copy": round(2 * io / (tsb - tsf) / 1e6 / copy_gbs, 3)}
 
 
-def generic_measurement(dev, gen):
-    """The generic kernels (head dim 256; fp32 inputs) on the query-sparse
-    path: fwd+bwd effective TFLOP/s (selected rows only, as the headline) at
+def wide_fp32_measurement(dev, gen):
+    """Head dim 256 and fp32 inputs, which have kernels of their own, on the
+    query-sparse path: fwd+bwd effective TFLOP/s (selected rows only, as the headline) at
     T=8192, H=16, Markov r=0.25, for K=V=256 in bf16 and for D=128 in fp32
     (against the fp32 MFMA peak), and config 1 (B=1, H=4, T=512, D=64, fp32,
     Bernoulli 0.5) in ms."""
@@ -331,7 +331,7 @@ def extra_measurements(dev):
     out["cfg3_fwd_bwd_varlen"] = {"lens": lens, "ms": round(t3, 3), "tflops": round(f3 / t3 / 1e9, 1)}
 
     out["swa_w128_cfg4"] = swa_cfg4_measurement(q, k, v, do)
-    out["generic_kernels"] = generic_measurement(dev, gen)
+    out["wide_fp32"] = wide_fp32_measurement(dev, gen)
     N4 = 4 * 8192
 
     # fused epilogue at cfg4 shape: L, G [32768, 16, 128], gate [32768]
@@ -610,10 +610,10 @@ def main():
     if args.layer:
         print(json.dumps(layer_cfg4_measurement(dev)), flush=True)
         return
-    if args.generic:
+    if args.wide_fp32:
         g = torch.Generator()
         g.manual_seed(7)
-        print(json.dumps(generic_measurement(dev, g)), flush=True)
+        print(json.dumps(wide_fp32_measurement(dev, g)), flush=True)
         return
     if args.swa:
         g = torch.Generator()
