@@ -185,13 +185,13 @@ size_t logo_sq_kv_workspace_bytes(int64_t n_tokens, int nseq, int hq, int h, int
  */
 size_t logo_sq_wide_workspace_bytes(int hq);
 /* Fewest keys of a piece there: calls of fewer than twice as many tokens need no workspace. */
-#define LOGO_WIDE_SPLIT_KEYS 448
+#define LOGO_WIDE_SPLIT_KEYS 320
 /*
  * The forward of segments that are shorter on average runs on the generic
  * kernels, whose 16-row tiles and 32-key steps start sooner, without a workspace.
  * The others' time over theirs, mean and worst over 1 to 16 heads and 5 to 40 % of
- * the rows: one segment of 300 tokens 1.00, 1.14, of 500 0.89, 0.96; six segments
- * of 333 tokens 1.03, 1.36, of 500 0.85, 1.07.
+ * the rows: one segment of 300 tokens 1.00, 1.14, of 500 0.88, 0.93; six segments
+ * of 333 tokens 1.03, 1.36, of 500 0.84, 1.15.
  */
 #define LOGO_WIDE_FWD_MIN_TOKENS 352
 

@@ -49,9 +49,7 @@ struct AttnArgs {
   float* part;
   int* cnt;
   int split_cap;
-  // fewest keys of a piece, where all pieces run at once and where they take turns
-  // on the CUs (0: the 64-key alignment alone)
-  int split_keys, split_keys_turns;
+  int split_keys;  // fewest keys of a piece (0: the 64-key alignment alone)
   // the caller's workspace (host side only: the launchers carve part / cnt
   // from it when it is large enough for their kernel's split_cap)
   void* ws;
@@ -376,8 +374,7 @@ struct QTile {
     if (nper > 1) {
       // 64-key-aligned chunks; nsplit <= nper pieces, none empty
       const int span = kv_hi - kv_lo;
-      const int least = 2 * nt * nper <= a.split_cap ? a.split_keys : a.split_keys_turns;
-      const int most = least > 0 ? max(1, min(nper, span / least)) : nper;
+      const int most = a.split_keys > 0 ? max(1, min(nper, span / a.split_keys)) : nper;
       const int chunk = (((span + most - 1) / most) + 63) & ~63;
       nsplit = (span + chunk - 1) / chunk;
       if (piece >= nsplit) return false;

@@ -888,11 +888,11 @@ int launch_rows(const AttnArgs& a_in, hipStream_t st, bool bwd) {
   AttnArgs a = a_in;
   split_setup(a, 1, bwd ? dq_part_floats(D) : fwd_part_floats(D, 4));
   // A piece starts with the loads of its rows and leaves 133 KB of partials: about
-  // the time of 400 keys.  Without a least size, forward and backward of 3000 and
-  // 4000 tokens in six segments (1 to 16 heads, 5 to 40 % of the rows) took up to
-  // 1.06x of the generic kernels' time, up to 0.89x so.
+  // the time of 400 keys.  Time over the generic kernels', forward and backward of
+  // 500 to 8192 tokens in one and six segments, 4 to 32 heads, 5 to 60 % of the rows:
+  // 0.622x with at least 320 keys (256: 0.623x; 448, and 1024 where the pieces take
+  // turns on the CUs: 0.633x); 0.655x without a least size, up to 1.34x.
   a.split_keys = LOGO_WIDE_SPLIT_KEYS;
-  a.split_keys_turns = 1024;
   a.round_rows /= 2;  // one 128-row workgroup per CU in a round
   const int64_t nblk = std::max<int64_t>((a.n + kBQ - 1) / kBQ + a.nseq, 2 * a.split_cap) * a.hq;
   LOGO_REQUIRE(nblk < ((int64_t)1 << 31), "grid too large");

@@ -69,8 +69,8 @@ def test_tile_edges_beside_a_long_segment(gpu, lens):
     ([513, 200], 2, 1, 0.4, False, torch.float16),
     ([300, 301], 2, 1, None, False, torch.bfloat16),  # dense rows
     ([1100], 8, 4, 0.02, False, torch.bfloat16),      # few rows
-    ([895], 2, 2, 0.6, False, torch.bfloat16),        # one key fewer than is cut, and the fewest that are
-    ([896, 5], 2, 2, 0.6, False, torch.bfloat16),
+    ([639], 2, 2, 1.1, False, torch.bfloat16),        # one key fewer than is cut, and the fewest that are
+    ([640], 2, 2, 1.1, False, torch.bfloat16),
     ([4500], 16, 16, 0.13, False, torch.bfloat16),    # pieces that take turns on the CUs
 ])
 def test_longer_sequences(gpu, lens, hq, h, rows, per_head, dtype):
