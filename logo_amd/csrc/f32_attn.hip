@@ -20,7 +20,7 @@
 // All partial sums are added in a fixed order.
 // Measured against 16 rows or keys a wave, 64 a workgroup, no key or row groups:
 // T = 4096, 16 heads, D = 128, a quarter of the rows, forward + backward 1238 to
-// 1306 -> 715 to 802 us on the boxes measured; 512 tokens, 4 heads, D = 64: the
+// 1306 -> 715 to 821 us on the boxes measured; 512 tokens, 4 heads, D = 64: the
 // three kernels 34 + 42 + 36 -> 13 + 13 + 12 us.  At T = 8192 the matrix units are
 // 54 / 75 / 79% busy (forward, dq, dk/dv); the forward's waves meet at a barrier
 // every 16 keys and do their softmax together.  Running S of the next tile beside

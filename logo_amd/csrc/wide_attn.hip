@@ -17,7 +17,7 @@
 // the rows it waits 40 / 33 / 34% of its time (forward, dq, dk/dv: for barriers,
 // the copies behind them, LDS operands) with the matrix units 26 / 37 / 32%, the
 // VALU 20 / 16 / 25% and the LDS 13 / 19 / 22% busy.  Forward + backward there:
-// 806 to 897 us on the boxes measured, 1834 to 1866 on the generic kernels (16
+// 784 to 897 us on the boxes measured, 1825 to 1866 on the generic kernels (16
 // rows or keys a wave on 16x16 MFMAs, one LDS operand read per half as many FLOPs,
 // no pipelining); 4001 tokens, 4 heads, forward only with split key ranges: 70
 // against 227 us; a few hundred tokens are bound by the launches either way.
